@@ -5,19 +5,20 @@
 // (flash-attn's bottom-right causal alignment): a chunk of a long prompt
 // attends to the retained earlier chunks plus itself.
 //
-// bf16 in/out, fp32 softmax, GQA.  One workgroup = 64 query rows of one query
-// head (4 waves x 16 rows); key/value blocks of 64 tokens are staged in LDS
-// (K row-major, V transposed) and shared by the 4 waves.  Per wave:
-//   S^T (keys x queries) = K . Q^T   with v_mfma_f32_16x16x32_bf16
-//   online softmax in the log2 domain (row max across 4 lane groups)
-//   O (queries x d) += P . V         with v_mfma_f32_16x16x32_bf16
-// MFMA 16x16x32 bf16 operand layout (lane l, 8 values each):
-//   A[row = l%16][k = 8*(l/16) + i],  B[k = 8*(l/16) + i][col = l%16],
-//   C[row = 4*(l/16) + r][col = l%16], r = 0..3.
-// S^T's C layout gives lane l the scores of query l%16 for keys
-// 16t + 4*(l/16) + r, which is directly the A operand of P.V once the key
-// order inside each 32-key MFMA step is permuted the same way for V.
-#include <cstdlib>
+// bf16 in/out, fp32 softmax, GQA.  A workgroup takes 128 query rows -- P =
+// 128 / G positions of the G query heads that share a KV head (G = 1, 2, 4;
+// other group sizes run G = 1, one query head at a time) -- four waves of 32
+// rows.  Per 64-key block a wave computes, on v_mfma_f32_32x32x16_bf16,
+//   S^T (keys x queries) = K . Q^T,   p = exp2(S * scale - m),
+//   O^T (d x queries)   += V^T . P^T.
+// Operand layout (lane l, half = l / 32, 8 values i each):
+//   A[row = l % 32][k = 8 * half + i],  B[k = 8 * half + i][col = l % 32],
+//   C[row = 8 * (r / 4) + 4 * half + r % 4][col = l % 32], r = 0 .. 15.
+// A lane owns one query: its max, its sum and its rescale factor are scalars
+// of that lane (one half swap per block, no broadcasts).  S^T's C layout is
+// the B operand of V^T . P^T once the 16 keys of a step are taken in the order
+// 8 * (i / 4) + 4 * half + i % 4, which is the order V is read in.
+#include <type_traits>
 
 #include "fdms_common.h"
 
@@ -26,12 +27,14 @@ using namespace fdms;
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kQRows = 64;   // query rows per workgroup
 constexpr int kKeys = 64;    // keys per LDS block
 constexpr int kThreads = 256;
+constexpr int kWaveRows = 32;  // query rows per wave
 
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
   bf16x8 r;
@@ -39,225 +42,100 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
   return r;
 }
 
-__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
-  return f32_to_bf16(a) | (f32_to_bf16(b) << 16);
-}
-
 // Two fp32 -> bf16 (round to nearest even) in one v_cvt_pk_bf16_f32.
 __device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  const bf16x2_t r = {(__bf16)a, (__bf16)b};
+  const bf16x2 r = {(__bf16)a, (__bf16)b};
   return __builtin_bit_cast(uint32_t, r);
 }
 
 __device__ __forceinline__ f32x4 mfma16x16x32(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ f32x16 mfma32x32x16(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// 16 bytes per lane from base + voff straight into LDS at lds + 16 * lane
+// (lds wave-uniform).  The compiler does not count it: lds_dma_barrier() below
+// waits for it before the workgroup's barrier.
+__device__ __forceinline__ void lds_dma16(const uint8_t* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+// Every LDS-DMA of this wave has landed and every LDS read of it has
+// returned, then the workgroup's barrier.
+__device__ __forceinline__ void lds_dma_barrier() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Max over the two lanes of a query (l and l ^ 32).
+__device__ __forceinline__ float halves_max(float v) {
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __builtin_elementwise_maximum(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float halves_sum(float v) {
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
 
 }  // namespace
 
-// FASTDMS_AMD_PREFILL_GQA=0 selects the per-head kernel for every shape
-// (comparison / testing).
-static bool fdms_prefill_gqa_enabled() {
-  static const bool on = [] {
-    const char* e = std::getenv("FASTDMS_AMD_PREFILL_GQA");
-    return !(e && e[0] == '0');
-  }();
-  return on;
-}
-
-template <int D>
-__global__ __launch_bounds__(kThreads) void prefill_attn_kernel(
+// K/V blocks go from global memory straight into LDS, row-major and unpadded
+// with the 16-byte chunks of a row XOR-swizzled (the lane picks which chunk it
+// loads), double-buffered.  K: chunk c of row r at slot c ^ (r & 15) (head_dim
+// 128; (r / 2) & 7 at 64), so the 32 rows of an A operand spread over all
+// banks.  V: chunk c at slot c ^ 4 * (r & 3) (4 * ((r / 2) & 1)); its A operand is
+// read with the transposing ds_read_b64_tr_b16 (16 lanes: four keys x 16 dims).
+//
+// What bounds it: power and the matrix cores together -- the clock falls to
+// 1.8 GHz while it runs (2.35 GHz under a memory-bound kernel) with the matrix
+// cores 51 % (head_dim 64) / 59 % (128) and the VALU 73 % / 46 % busy -- so what
+// counts is work per score.  32 rows per wave in 32x32 tiles keep two waves per
+// SIMD at head_dim 128 and three at 64 (227 / 159 VGPRs); the direct LDS loads
+// and the transposing reads take the V transposition and the staging registers
+// away, one lane per query the softmax broadcasts, and v_dot2 the extra P . 1
+// tile.  Measured against 16x16 tiles staged through registers: eight ragged
+// prompts of 6 144 tokens, 32 / 8 heads, head_dim 64 1 670 -> 1 380 us (929
+// TFLOP/s), head_dim 128 3 197 -> 2 428 us (1 059); 4 096 queries over a 12 300
+// token prefix, head_dim 128 1 128 -> 854 us (1 134); 24 prompts of 400 tokens
+// 46 -> 34.6 us.  P.V delayed by a block (so that one straight-line region holds
+// both products and the exponentials) measured +2 % / -0.5 %, and replacing
+// the per-block max by a check of the running sum -2.7 % at head_dim 64 but +1 to
+// +5 % at 128.
+//
+// Software pipeline over the blocks: iteration t holds S of block t, issues
+// the loads of K(t + 2) and V(t + 1), multiplies K(t + 1) . Q^T beside the
+// exponentials of block t, then V(t) . P beside the max of block t + 1.
+// Softmax rescaling is lazy: the running max only moves (and O / the sum are
+// rescaled) when a block raises it by more than 8 in the log2 domain, so p
+// stays below 256.  The running max starts at a finite floor (-1e30) instead
+// of -inf: the first block with a visible key then takes the same grow test
+// as every later one, its rescale factor exp2((floor - m) * scale) is exactly 0,
+// and a row whose keys so far are all masked keeps the floor with p = 0.
+template <int D, int G>
+__global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
     const bf16_t* __restrict__ q, int64_t qs_t, int64_t qs_h, const bf16_t* __restrict__ k, int64_t ks_t,
     int64_t ks_h, const bf16_t* __restrict__ v, int64_t vs_t, int64_t vs_h, bf16_t* __restrict__ out, int64_t os_t,
-    int64_t os_h, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, int group,
+    int64_t os_h, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, int group, int vec_out,
     float scale_log2) {
-  constexpr int KPAD = D + 8;       // sK row stride (bf16)
-  constexpr int VPAD = kKeys + 8;   // sVt row stride (bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t sK[kKeys * KPAD];
-  __shared__ __attribute__((aligned(16))) uint16_t sVt[D * VPAD];
+  constexpr int P = 4 * kWaveRows / G;  // query positions per workgroup
+  constexpr int RB = 2 * D;             // bytes of a K / V row
+  constexpr int CH = D / 8;             // 16-byte chunks of a row
+  constexpr int TILE = kKeys * RB;
+  constexpr int RPI = 1024 / RB;        // rows one wave's LDS-DMA instruction moves
+  constexpr int NI = kKeys / (4 * RPI);  // such instructions per wave and tile
+  constexpr int KS = D / 16;            // MFMA steps of QK^T
+  constexpr int DT = D / 32;            // 32-dim tiles of O^T
+  __shared__ __attribute__((aligned(1024))) uint8_t s_kv[4 * TILE];  // K0, K1, V0, V1
 
+  // block ids run over (head group, query block) with the head group fastest,
+  // so with 8 KV heads every XCD (ids go round-robin over them) keeps one
+  // head's K / V in its L2; a head's heaviest (diagonal-last) blocks go first
   const int seq = blockIdx.z;
-  const int qh = blockIdx.y;
-  const int kvh = qh / group;
-  // query rows are the last qlen of the sequence's klen keys (bottom-right
-  // causal alignment): row i is position off + i and sees keys 0 .. off + i
-  const int start = cu_q[seq];
-  const int len = cu_q[seq + 1] - start;
-  const int kstart = cu_k[seq];
-  const int klen = cu_k[seq + 1] - kstart;
-  const int off = klen - len;
-  if (off < 0) return;  // rejected: more queries than keys
-  const int nqb = (len + kQRows - 1) / kQRows;
-  if ((int)blockIdx.x >= nqb) return;
-  const int qb = nqb - 1 - (int)blockIdx.x;  // heaviest (diagonal-last) blocks first
-  const int q0 = qb * kQRows;
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const int lg = lane >> 4;   // lane group 0..3
-  const int lc = lane & 15;   // lane column 0..15
-  const int my_q = q0 + wave * 16 + lc;  // query row this lane's S^T column belongs to
-
-  // Q^T as the B operand of S^T = K.Q^T: lane holds Q[my_q][32j + 8*lg + i]
-  bf16x8 qop[D / 32];
-  {
-    const int qrow = min(my_q, len - 1);
-    const bf16_t* qp = q + (int64_t)(start + qrow) * qs_t + (int64_t)qh * qs_h;
-#pragma unroll
-    for (int j = 0; j < D / 32; ++j) qop[j] = as_bf16x8(*reinterpret_cast<const uint4*>(qp + 32 * j + 8 * lg));
-  }
-
-  float m_run = -INFINITY;  // running max of query my_q (same in the 4 lane groups)
-  float l_part = 0.0f;      // this lane's partial softmax denominator
-  f32x4 o[D / 16];          // O[q = 4*lg + r][d = 16c + lc] of this wave's 16 rows
-#pragma unroll
-  for (int c = 0; c < D / 16; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int nkb = min((klen + kKeys - 1) / kKeys, (off + q0 + kQRows - 1) / kKeys + 1);
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int k0 = kb * kKeys;
-    __syncthreads();
-    // stage K (row-major) and V (transposed) for keys k0..k0+63; zero beyond len
-    for (int u = tid; u < kKeys * D / 8; u += kThreads) {
-      const int key = u / (D / 8);
-      const int d0 = (u - key * (D / 8)) * 8;
-      uint4 kv = {0u, 0u, 0u, 0u}, vv = {0u, 0u, 0u, 0u};
-      if (k0 + key < klen) {
-        kv = *reinterpret_cast<const uint4*>(k + (int64_t)(kstart + k0 + key) * ks_t + (int64_t)kvh * ks_h + d0);
-        vv = *reinterpret_cast<const uint4*>(v + (int64_t)(kstart + k0 + key) * vs_t + (int64_t)kvh * vs_h + d0);
-      }
-      *reinterpret_cast<uint4*>(&sK[key * KPAD + d0]) = kv;
-      const uint16_t* vh = reinterpret_cast<const uint16_t*>(&vv);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) sVt[(d0 + i) * VPAD + key] = vh[i];
-    }
-    __syncthreads();
-
-    // S^T for the 4 key tiles of 16: lane gets keys 16t + 4*lg + r for query my_q
-    float s[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j < D / 32; ++j) {
-        const bf16x8 a = as_bf16x8(*reinterpret_cast<const uint4*>(&sK[(16 * t + lc) * KPAD + 32 * j + 8 * lg]));
-        acc = mfma16x16x32(a, qop[j], acc);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = k0 + 16 * t + 4 * lg + r;
-        const bool ok = key <= off + my_q && key < klen;
-        s[t][r] = ok ? acc[r] * scale_log2 : -INFINITY;
-      }
-    }
-    float bmax = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) bmax = fmaxf(bmax, s[t][r]);
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 16));
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32));
-    const float m_new = fmaxf(m_run, bmax);
-    const float alpha = (m_run == -INFINITY) ? 0.0f : exp2f(m_run - m_new);
-    m_run = m_new;
-    float psum = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = (s[t][r] == -INFINITY) ? 0.0f : exp2f(s[t][r] - m_new);
-        s[t][r] = p;
-        psum += p;
-      }
-    l_part = l_part * alpha + psum;
-    // rescale O rows q = 4*lg + r by alpha of that query (held by lane 4*lg + r)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float ar = __shfl(alpha, 4 * lg + r);
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c) o[c][r] *= ar;
-    }
-    // O += P.V over two 32-key steps; k index i of lane group lg = key 32*st + 16*(i/4) + 4*lg + i%4
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      uint4 pa;
-      pa.x = pack_bf16x2(s[2 * st][0], s[2 * st][1]);
-      pa.y = pack_bf16x2(s[2 * st][2], s[2 * st][3]);
-      pa.z = pack_bf16x2(s[2 * st + 1][0], s[2 * st + 1][1]);
-      pa.w = pack_bf16x2(s[2 * st + 1][2], s[2 * st + 1][3]);
-      const bf16x8 a = as_bf16x8(pa);
-      const int key_a = 32 * st + 4 * lg;
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c) {
-        const uint16_t* vr = &sVt[(16 * c + lc) * VPAD];
-        uint4 b;
-        const uint2 lo = *reinterpret_cast<const uint2*>(vr + key_a);
-        const uint2 hi = *reinterpret_cast<const uint2*>(vr + key_a + 16);
-        b.x = lo.x;
-        b.y = lo.y;
-        b.z = hi.x;
-        b.w = hi.y;
-        o[c] = mfma16x16x32(a, as_bf16x8(b), o[c]);
-      }
-    }
-  }
-
-  float l_tot = l_part;
-  l_tot += __shfl_xor(l_tot, 16);
-  l_tot += __shfl_xor(l_tot, 32);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float inv = 1.0f / __shfl(l_tot, 4 * lg + r);
-    const int row = q0 + wave * 16 + 4 * lg + r;
-    if (row < len) {
-      bf16_t* op = out + (int64_t)(start + row) * os_t + (int64_t)qh * os_h;
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c) op[16 * c + lc].bits = (uint16_t)f32_to_bf16(o[c][r] * inv);
-    }
-  }
-}
-
-// GQA-packed variant for group sizes 1, 2 and 4: a workgroup takes P =
-// 64·QT/G query positions of one KV head for all G query heads that share it,
-// so one staged K/V block feeds 64·QT query rows (wave w: head w % G,
-// positions 16·QT·(w / G) .. +16·QT-1, QT 16-row MFMA tiles; QT = 2: QT = 4
-// halves the LDS reads per MFMA but costs an occupancy step (3 -> 2 waves per
-// SIMD at head_dim 64) and measured no faster).  K/V blocks of 64 keys are
-// double-buffered in LDS: the next block's global loads are in flight while
-// the current one is computed, and one barrier separates blocks.  V is
-// transposed in registers (4 keys x 8 dims per thread, byte permutes) so the
-// LDS stores are 8-byte vectors.  Every K fragment read from LDS feeds both
-// query tiles of a wave, as does every V fragment.  The softmax row sums come
-// from the matrix cores (P . 1, an extra output tile).  Softmax rescaling is
-// lazy: the running max only moves (and O / the sums are rescaled) when a block raises it
-// by more than 8 in the log2 domain, so p = exp2(s - m) stays below 256.  The
-// running max starts at a finite floor (-1e30) instead of -inf: the first
-// block with a visible key then takes the same grow test as every later one,
-// its rescale factor exp2((floor - m) * scale) is exactly 0, and a row whose
-// keys so far are all masked keeps the floor with p = exp2(-inf) = 0 -- the
-// same results as special-casing -inf, with fewer VALU instructions per block.
-template <int D, int G, int QT>
-__global__ __launch_bounds__(kThreads) void prefill_attn_gqa_kernel(
-    const bf16_t* __restrict__ q, int64_t qs_t, int64_t qs_h, const bf16_t* __restrict__ k, int64_t ks_t,
-    int64_t ks_h, const bf16_t* __restrict__ v, int64_t vs_t, int64_t vs_h, bf16_t* __restrict__ out, int64_t os_t,
-    int64_t os_h, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, float scale_log2) {
-  constexpr int RW = 16 * QT;       // query rows per wave (QT 16-row MFMA tiles)
-  constexpr int P = 4 * RW / G;     // query positions per workgroup
-  constexpr int KPAD = D + 8;       // sK row stride (bf16)
-  // sVt row stride (bf16): 136 B = 34 dwords, so the 16 lanes of one 8-byte
-  // B-operand read (rows 16c + lc) land on 16 distinct bank pairs
-  constexpr int VPAD = kKeys + 4;
-  constexpr int UNITS = 4 * D;      // staging units per block: 2D V quads (4 keys x 8 dims) + 2D K quads (4 chunks)
-  constexpr int UPT = UNITS / kThreads;
-  static_assert(UNITS % kThreads == 0, "staging units must divide over the workgroup");
-  __shared__ __attribute__((aligned(16))) uint16_t sK[2][kKeys * KPAD];
-  __shared__ __attribute__((aligned(16))) uint16_t sVt[2][D * VPAD];
-
-  const int seq = blockIdx.z;
-  const int kvh = blockIdx.y;
+  const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y;
+  const int hg = (int)(lin % gridDim.y), qb = (int)(lin / gridDim.y);
   // query rows are the last len of the klen keys (bottom-right causal
-  // alignment, as the per-head kernel); positions below are query rows
+  // alignment): row i is position off + i and sees keys 0 .. off + i
   const int start = cu_q[seq];
   const int len = cu_q[seq + 1] - start;
   const int kstart = cu_k[seq];
@@ -265,219 +143,231 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_gqa_kernel(
   const int off = klen - len;
   if (off < 0) return;  // rejected: more queries than keys
   const int nqb = (len + P - 1) / P;
-  if ((int)blockIdx.x >= nqb) return;
-  const int q0 = (nqb - 1 - (int)blockIdx.x) * P;  // heaviest (diagonal-last) blocks first
+  if (qb >= nqb) return;
+  const int q0 = (nqb - 1 - qb) * P;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  const int lg = lane >> 4;
-  const int lc = lane & 15;
-  const int qh = kvh * G + wave % G;
-  const int wq0 = q0 + (wave / G) * RW;            // first position of this wave
-  const int wq_last = min(wq0 + RW - 1, len - 1);  // last valid position of this wave
+  const int lc = lane & 31, half = lane >> 5;
+  const int qh = hg * G + wave % G;
+  const int kvh = (hg * G) / group;
+  const int wq0 = q0 + (wave / G) * kWaveRows;                  // first position of this wave
+  const int wq_last = min(wq0 + kWaveRows - 1, len - 1);        // last valid position of this wave
+  const int kend = min(klen, off + q0 + P);                     // keys some row of the workgroup sees
+  const int nkb = (kend + kKeys - 1) / kKeys;
+  const int nw = wq0 < len ? (off + wq_last) / kKeys + 1 : 0;   // blocks this wave sees (<= nkb)
 
-  bf16x8 qop[QT][D / 32];
+  const uint8_t* kbase = reinterpret_cast<const uint8_t*>(k + (int64_t)kstart * ks_t + (int64_t)kvh * ks_h);
+  const uint8_t* vbase = reinterpret_cast<const uint8_t*>(v + (int64_t)kstart * vs_t + (int64_t)kvh * vs_h);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)s_kv;
+  // this lane's part of an LDS-DMA instruction: row drow (+ 4 * RPI * i), the
+  // chunk whose swizzled slot is lane % CH
+  const int drow = wave * RPI + lane / CH;
+  const int kchunk = (lane % CH) ^ (D == 128 ? drow & 15 : (drow >> 1) & 7);
+  const int vchunk = (lane % CH) ^ (D == 128 ? (drow & 3) << 2 : ((drow >> 1) & 1) << 2);
+  const uint32_t ksb = (uint32_t)(ks_t * 2), vsb = (uint32_t)(vs_t * 2);  // row strides in bytes
+  auto load_tile = [&](const uint8_t* base, uint32_t stride, int chunk, int blk, uint32_t lds) {
+    const int k0 = blk * kKeys;
+    const uint8_t* b = base + (int64_t)k0 * stride;
+    const int last = klen - 1 - k0;  // rows past the sequence end repeat its last (their scores are masked)
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt) {
-    const int qrow = min(wq0 + 16 * qt + lc, len - 1);
-    const bf16_t* qp = q + (int64_t)(start + qrow) * qs_t + (int64_t)qh * qs_h;
-#pragma unroll
-    for (int j = 0; j < D / 32; ++j) qop[qt][j] = as_bf16x8(*reinterpret_cast<const uint4*>(qp + 32 * j + 8 * lg));
-  }
+    for (int i = 0; i < NI; ++i)
+      lds_dma16(b, (uint32_t)min(drow + 4 * RPI * i, last) * stride + 16 * chunk,
+                lds + (uint32_t)((i * 4 + wave) * 1024));
+  };
+  auto load_k = [&](int blk, int buf) { load_tile(kbase, ksb, kchunk, blk, lds0 + buf * TILE); };
+  auto load_v = [&](int blk, int buf) { load_tile(vbase, vsb, vchunk, blk, lds0 + (2 + buf) * TILE); };
 
-  const bf16_t* kb_base = k + (int64_t)kstart * ks_t + (int64_t)kvh * ks_h;
-  const bf16_t* vb_base = v + (int64_t)kstart * vs_t + (int64_t)kvh * vs_h;
-  uint4 stage[UPT][4];
-  // unit u < 2D: V quad (keys 4*(u % 16) .. +3, dims 8*(u / 16) .. +7: the 16
-  // lanes of a row store 128 contiguous bytes of one transposed row);
-  // u >= 2D: K chunks (u - 2D) + 2D*r, r = 0..3 (chunk c = key * (D/8) + dim / 8:
-  // consecutive lanes move consecutive 16-byte chunks).
-  // Row r of unit i is key k0 + krow[i][r] at element offset koff[i][r] +
-  // key * stride; rows past the sequence end are clamped (their scores are
-  // masked).
-  // Whether unit i is a V or a K unit is uniform per wave (2D is a multiple
-  // of 64), so a block's row base is a scalar and each lane adds a fixed
-  // 32-bit element offset: the loads of a block cost no vector address math.
-  int krow[UPT][4], koff[UPT][4], eoff[UPT][4];
-  const bf16_t* kvp[UPT];
-  int64_t kvs[UPT];
+  load_k(0, 0);
+  load_v(0, 0);
+  if (nkb > 1) load_k(1, 1);
+  bf16x8 qop[KS];
+  {
+    const int qrow = min(wq0 + lc, len - 1);
+    const bf16_t* qp = q + (int64_t)(start + qrow) * qs_t + (int64_t)qh * qs_h + 8 * half;
 #pragma unroll
-  for (int i = 0; i < UPT; ++i) {
-    const int u = tid + i * kThreads;
-    const bool is_v = __builtin_amdgcn_readfirstlane((int)(u < 2 * D)) != 0;
-    kvp[i] = is_v ? vb_base : kb_base;
-    kvs[i] = is_v ? vs_t : ks_t;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int c = (u - 2 * D) + 2 * D * r;
-      krow[i][r] = is_v ? 4 * (u % 16) + r : c / (D / 8);
-      koff[i][r] = is_v ? 8 * (u / 16) : 8 * (c % (D / 8));
-      eoff[i][r] = krow[i][r] * (int)kvs[i] + koff[i][r];  // < 64 rows: within int range for any real stride
-    }
+    for (int j = 0; j < KS; ++j) qop[j] = as_bf16x8(*reinterpret_cast<const uint4*>(qp + 16 * j));
   }
-  auto load_block = [&](int k0) {
-    if (k0 + kKeys <= klen) {  // uniform
+  // LDS byte offsets of this lane's operands (buffer, key tile and key step
+  // are added as constants)
+  uint32_t kaddr[KS], vaddr[DT];
 #pragma unroll
-      for (int i = 0; i < UPT; ++i) {
-        const bf16_t* base = kvp[i] + (int64_t)k0 * kvs[i];  // scalar
+  for (int j = 0; j < KS; ++j)
+    kaddr[j] = lc * RB + (((2 * j + half) ^ (D == 128 ? lc & 15 : (lc >> 1) & 7)) << 4);
+  {
+    const int l16 = lane & 15, g1 = (lane >> 4) & 1;
+    const int vr = 4 * half + (l16 >> 2);
+    const int f = D == 128 ? (vr & 3) << 2 : ((vr >> 1) & 1) << 2;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) stage[i][r] = *reinterpret_cast<const uint4*>(base + eoff[i][r]);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < UPT; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = min(k0 + krow[i][r], klen - 1);  // rows past the end clamped (their scores are masked)
-          stage[i][r] = *reinterpret_cast<const uint4*>(kvp[i] + (int64_t)key * kvs[i] + koff[i][r]);
-        }
-    }
-  };
-  auto store_block = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < UPT; ++i) {
-      const int u = tid + i * kThreads;
-      if (u < 2 * D) {
-        const int kq = u % 16, dc = u / 16;
-        const uint32_t w0[4] = {stage[i][0].x, stage[i][0].y, stage[i][0].z, stage[i][0].w};
-        const uint32_t w1[4] = {stage[i][1].x, stage[i][1].y, stage[i][1].z, stage[i][1].w};
-        const uint32_t w2[4] = {stage[i][2].x, stage[i][2].y, stage[i][2].z, stage[i][2].w};
-        const uint32_t w3[4] = {stage[i][3].x, stage[i][3].y, stage[i][3].z, stage[i][3].w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-          uint2 t;
-          t.x = __builtin_amdgcn_perm(w1[e >> 1], w0[e >> 1], sel);  // keys 4kq, 4kq+1 of dim 8dc+e
-          t.y = __builtin_amdgcn_perm(w3[e >> 1], w2[e >> 1], sel);  // keys 4kq+2, 4kq+3
-          *reinterpret_cast<uint2*>(&sVt[buf][(8 * dc + e) * VPAD + 4 * kq]) = t;
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int c = (u - 2 * D) + 2 * D * r;
-          *reinterpret_cast<uint4*>(&sK[buf][(c / (D / 8)) * KPAD + 8 * (c % (D / 8))]) = stage[i][r];
-        }
-      }
-    }
-  };
+    for (int c = 0; c < DT; ++c)
+      vaddr[c] = vr * RB + (((4 * c + 2 * g1 + ((l16 & 3) >> 1)) ^ f) << 4) + 8 * (l16 & 1);
+  }
 
   constexpr float kMaxFloor = -1e30f;  // below any score; see the rescale note above
-  float m_run[QT];  // raw-score running max of query lc of each tile
+  float m_run = kMaxFloor;             // raw-score running max of this lane's query
+  float l_run = 0.0f;                  // this half's share of its row sum
+  f32x16 o[DT];
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt) m_run[qt] = kMaxFloor;
-  // o[qt][D/16] accumulates P . 1 on the matrix cores: column-replicated row
-  // sums of the same bf16 P as the numerator, in the O layout (no shuffles)
-  f32x4 o[QT][D / 16 + 1];
-#pragma unroll
-  for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-    for (int c = 0; c <= D / 16; ++c) o[qt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bf16x8 ones = as_bf16x8(uint4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+  for (int c = 0; c < DT; ++c) o[c] = f32x16{};
+  f32x16 s0[2], s1[2];
+  const int lim = off + min(wq0 + lc, len - 1) - 4 * half;  // last visible key - 4 * half
 
-  const int kend = min(klen, off + q0 + P);  // keys 0 .. kend-1 are visible to some row of the workgroup
-  const int nkb = (kend + kKeys - 1) / kKeys;
-  load_block(0);
-  store_block(0);
-  __syncthreads();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int k0 = kb * kKeys;
-    const int buf = kb & 1;
-    const bool more = kb + 1 < nkb;
-    if (more) load_block(k0 + kKeys);
-    if (k0 <= off + wq_last) {  // wave-uniform: this block holds keys visible to the wave
-      f32x4 acc[QT][4];
+  auto qk = [&](f32x16 (&sx)[2], int buf) {
+    const uint8_t* kt = s_kv + buf * TILE;
+    sx[0] = sx[1] = f32x16{};
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+    for (int j = 0; j < KS; ++j) {
+      const bf16x8 a0 = as_bf16x8(*reinterpret_cast<const uint4*>(kt + kaddr[j]));
+      const bf16x8 a1 = as_bf16x8(*reinterpret_cast<const uint4*>(kt + 32 * RB + kaddr[j]));
+      sx[0] = mfma32x32x16(a0, qop[j], sx[0]);
+      sx[1] = mfma32x32x16(a1, qop[j], sx[1]);
+    }
+  };
+  auto mask = [&](f32x16 (&sx)[2], int blk) {
+    const int rel = lim - blk * kKeys;
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) acc[qt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int j = 0; j < D / 32; ++j) {
-          const bf16x8 a = as_bf16x8(*reinterpret_cast<const uint4*>(&sK[buf][(16 * t + lc) * KPAD + 32 * j + 8 * lg]));
+      for (int r = 0; r < 16; ++r) sx[t][r] = 32 * t + 8 * (r / 4) + r % 4 > rel ? -INFINITY : sx[t][r];
+  };
+  // NaN-propagating max (one instruction per two scores): a row with a NaN
+  // score is NaN whatever its max is
+  auto row_max = [&](const f32x16 (&sx)[2]) {
+    float b0 = __builtin_elementwise_maximum(sx[0][0], sx[1][0]);
+    float b1 = __builtin_elementwise_maximum(sx[0][1], sx[1][1]);
 #pragma unroll
-          for (int qt = 0; qt < QT; ++qt) acc[qt][t] = mfma16x16x32(a, qop[qt][j], acc[qt][t]);
-        }
+    for (int r = 2; r < 16; r += 2) {
+      b0 = __builtin_elementwise_maximum(__builtin_elementwise_maximum(b0, sx[0][r]), sx[1][r]);
+      b1 = __builtin_elementwise_maximum(__builtin_elementwise_maximum(b1, sx[0][r + 1]), sx[1][r + 1]);
+    }
+    return halves_max(__builtin_elementwise_maximum(b0, b1));
+  };
+  auto rescale = [&](float bmax) {
+    // lazy: move the max only when it grows by more than 2^8 in p
+    const bool grow = (bmax - m_run) * scale_log2 > 8.0f;  // bmax = -inf (all masked): false
+    if (__builtin_amdgcn_ballot_w64(grow)) {               // wave-uniform
+      const float m_new = fmaxf(m_run, bmax);
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2);  // 0 from the floor
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int c = 0; c < DT; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[c][r] *= alpha;
+    }
+  };
+  // p of block t as the B operands of its four 16-key steps, and their sum
+  // (of the bf16 values, as the numerator uses them)
+  auto probs = [&](const f32x16 (&sx)[2], uint4 (&pb)[4]) {
+    const float mb = m_run * scale_log2;
+    const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 8 * (st & 1) + 2 * i;
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sx[st >> 1][r], scale_log2, -mb));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sx[st >> 1][r + 1], scale_log2, -mb));
+        w[i] = cvt_pk_bf16(p0, p1);
+        l_run = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w[i]), one, l_run, false);
       }
-      const bool masked = k0 + kKeys - 1 > off + wq0 || k0 + kKeys > klen;  // wave-uniform
-      if (masked) {
+      pb[st] = uint4{w[0], w[1], w[2], w[3]};
+    }
+  };
+  auto pv = [&](const uint4 (&pb)[4], int buf) {
+    using lds_s16x4 = __attribute__((address_space(3))) s16x4;
+    const uint32_t vt = lds0 + (2 + buf) * TILE;
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-          const int lim = off + min(wq0 + 16 * qt + lc, len - 1);
+    for (int st = 0; st < 4; ++st)
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int key = k0 + 16 * t + 4 * lg + r;
-              acc[qt][t][r] = key > lim ? -INFINITY : acc[qt][t][r];
-            }
-        }
+      for (int c = 0; c < DT; ++c) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(vt + vaddr[c] + (16 * st) * RB));
+        const s16x4 hi =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(vt + vaddr[c] + (16 * st + 8) * RB));
+        const auto both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        o[c] = mfma32x32x16(__builtin_bit_cast(bf16x8, both), as_bf16x8(pb[st]), o[c]);
       }
-      uint4 pa[QT][2];
-#pragma unroll
-      for (int qt = 0; qt < QT; ++qt) {
-        float bmax = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) bmax = fmaxf(bmax, acc[qt][t][r]);
-        bmax = rows_max(bmax);
-        // lazy rescale: move the max only when it grows by more than 2^8 in p
-        const bool grow = (bmax - m_run[qt]) * scale_log2 > 8.0f;  // bmax = -inf (all masked): false
-        if (__builtin_amdgcn_ballot_w64(grow)) {  // wave-uniform
-          const float m_new = fmaxf(m_run[qt], bmax);
-          const float alpha = __builtin_amdgcn_exp2f((m_run[qt] - m_new) * scale_log2);  // 0 from the floor
-          m_run[qt] = m_new;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float ar = __shfl(alpha, 4 * lg + r);
-#pragma unroll
-            for (int c = 0; c <= D / 16; ++c) o[qt][c][r] *= ar;
-          }
-        }
-        const float mb = m_run[qt] * scale_log2;
-        float p[4][4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) p[t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[qt][t][r], scale_log2, -mb));
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          pa[qt][st].x = cvt_pk_bf16(p[2 * st][0], p[2 * st][1]);
-          pa[qt][st].y = cvt_pk_bf16(p[2 * st][2], p[2 * st][3]);
-          pa[qt][st].z = cvt_pk_bf16(p[2 * st + 1][0], p[2 * st + 1][1]);
-          pa[qt][st].w = cvt_pk_bf16(p[2 * st + 1][2], p[2 * st + 1][3]);
-        }
-      }
-      // O += P.V; k index i of lane group lg = key 32*st + 16*(i/4) + 4*lg + i%4
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        const int key_a = 32 * st + 4 * lg;
-#pragma unroll
-        for (int c = 0; c < D / 16; ++c) {
-          const uint16_t* vr = &sVt[buf][(16 * c + lc) * VPAD];
-          const uint2 lo = *reinterpret_cast<const uint2*>(vr + key_a);
-          const uint2 hi = *reinterpret_cast<const uint2*>(vr + key_a + 16);
-          const bf16x8 b = as_bf16x8(uint4{lo.x, lo.y, hi.x, hi.y});
-#pragma unroll
-          for (int qt = 0; qt < QT; ++qt) o[qt][c] = mfma16x16x32(as_bf16x8(pa[qt][st]), b, o[qt][c]);
-        }
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) o[qt][D / 16] = mfma16x16x32(as_bf16x8(pa[qt][st]), ones, o[qt][D / 16]);
+  };
+
+  // blocks every row of the wave sees whole: the others need the mask
+  const int nfull = min((off + wq0 + 1) / kKeys, klen / kKeys);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), known to the compiler: Q has landed, no use of it waits again
+  lds_dma_barrier();
+  if (nw > 0) {
+    qk(s0, 0);
+    if (nfull < 1) mask(s0, 0);
+    rescale(row_max(s0));
+  }
+  lds_dma_barrier();  // K(0) has been read by every wave: its buffer takes K(2)
+  // B = t & 1; cur = S(t), nxt receives S(t + 1)
+  auto full = [&](int t, auto parity, f32x16 (&cur)[2], f32x16 (&nxt)[2]) {
+    constexpr int B = decltype(parity)::value;
+    uint4 pb[4];
+    qk(nxt, 1 - B);
+    probs(cur, pb);
+    pv(pb, B);
+    rescale(row_max(nxt));
+  };
+  auto loads = [&](int t, auto parity) {
+    constexpr int B = decltype(parity)::value;
+    if (t + 2 < nkb) load_k(t + 2, B);
+    if (t + 1 < nkb) load_v(t + 1, 1 - B);
+  };
+  auto iteration = [&](int t, auto parity, f32x16 (&cur)[2], f32x16 (&nxt)[2]) {
+    constexpr int B = decltype(parity)::value;
+    loads(t, parity);
+    if (t < nw) {  // wave-uniform, as the branch below
+      uint4 pb[4];
+      probs(cur, pb);
+      pv(pb, B);
+      if (t + 1 < nw) {
+        qk(nxt, 1 - B);
+        mask(nxt, t + 1);
+        rescale(row_max(nxt));
       }
     }
-    if (more) store_block(buf ^ 1);
-    __syncthreads();
+    if (t + 1 < nkb) lds_dma_barrier();
+  };
+  const std::integral_constant<int, 0> even{};
+  const std::integral_constant<int, 1> odd{};
+  int t = 0;
+  for (; t + 2 < nfull; t += 2) {
+    loads(t, even);
+    full(t, even, s0, s1);
+    lds_dma_barrier();
+    loads(t + 1, odd);
+    full(t + 1, odd, s1, s0);
+    lds_dma_barrier();
+  }
+  for (; t < nkb; t += 2) {
+    iteration(t, even, s0, s1);
+    if (t + 1 < nkb) iteration(t + 1, odd, s1, s0);
   }
 
+  const float inv = 1.0f / halves_sum(l_run);
+  const int row = wq0 + lc;
+  // lane (lc, half) holds dims 32 c + 8 g + 4 half + 0 .. 3 of its query in o[c][4 g ..]
+  bf16_t* op = out + (int64_t)(start + min(row, len - 1)) * os_t + (int64_t)qh * os_h;
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt) {
+  for (int c = 0; c < DT; ++c) {
+    uint32_t w[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float inv = 1.0f / o[qt][D / 16][r];  // row sum of query 4*lg + r
-      const int row = wq0 + 16 * qt + 4 * lg + r;
-      if (row < len) {
-        bf16_t* op = out + (int64_t)(start + row) * os_t + (int64_t)qh * os_h;
+    for (int i = 0; i < 8; ++i) w[i] = cvt_pk_bf16(o[c][2 * i] * inv, o[c][2 * i + 1] * inv);
+    if (vec_out) {  // uniform: 16-byte rows; the halves swap quads so that a lane stores 8 dims at once
 #pragma unroll
-        for (int c = 0; c < D / 16; ++c) op[16 * c + lc].bits = (uint16_t)f32_to_bf16(o[qt][c][r] * inv);
+      for (int m = 0; m < 2; ++m) {
+        const auto x = __builtin_amdgcn_permlane32_swap(w[4 * m], w[4 * m + 2], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(w[4 * m + 1], w[4 * m + 3], false, false);
+        if (row < len)
+          *reinterpret_cast<uint4*>(op + 32 * c + 16 * m + 8 * half) = uint4{x[0], y[0], x[1], y[1]};
+      }
+    } else if (row < len) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int d = 32 * c + 8 * (i / 2) + 4 * half + 2 * (i & 1);
+        op[d].bits = (uint16_t)w[i];
+        op[d + 1].bits = (uint16_t)(w[i] >> 16);
       }
     }
   }
@@ -493,50 +383,25 @@ FDMS_EXPORT int fdms_prefill_attention_varlen(const void* q, int64_t qs_t, int64
   if (num_seqs == 0 || max_seqlen_q <= 0) return 0;
   if (!q || !k || !v || !out || !cu_seqlens_q || !cu_seqlens_k) return (int)hipErrorInvalidValue;
   if (num_seqs > 65535 || num_q_heads > 65535) return (int)hipErrorInvalidValue;
-  // token strides in elements: 64 rows of either stay in 32-bit offsets
+  // token strides in elements: 64 rows of either stay in 32-bit byte offsets
   if (ks_t < 0 || vs_t < 0 || ks_t >= (1 << 24) || vs_t >= (1 << 24)) return (int)hipErrorInvalidValue;
+  if (head_dim != 64 && head_dim != 128) return (int)hipErrorInvalidValue;
   const float sl2 = scale * 1.4426950408889634f;
   const int group = num_q_heads / num_kv_heads;
-  const int32_t* cq = cu_seqlens_q;
-  const int32_t* ck = cu_seqlens_k;
-  if ((group == 1 || group == 2 || group == 4) && (head_dim == 64 || head_dim == 128) &&
-      fdms_prefill_gqa_enabled()) {
-    // 16-row query tiles per wave.  Four (head_dim 64 only) measured within
-    // 1 % of two on the Llama-3.2-1B c=8 prompts and 15 % slower on one
-    // 8192-token prompt, so two is the default
-    int qt = 2;
-    if (const char* e = std::getenv("FASTDMS_AMD_PREFILL_QT")) {  // comparison / testing
-      if (e[0] == '4' && head_dim == 64) qt = 4;
-    }
-    const int pos = 64 * qt / group;  // query positions per workgroup
-    const dim3 ggrid((max_seqlen_q + pos - 1) / pos, num_kv_heads, num_seqs);
-#define FDMS_PREFILL_GQA(DD, GG, QQ)                                                                               \
-  hipLaunchKernelGGL((prefill_attn_gqa_kernel<DD, GG, QQ>), ggrid, dim3(kThreads), 0, (hipStream_t)stream,          \
-                     (const bf16_t*)q, qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h,       \
-                     (bf16_t*)out, os_t, os_h, cq, ck, sl2)
-    if (head_dim == 64 && qt == 4) {
-      if (group == 1) FDMS_PREFILL_GQA(64, 1, 4); else if (group == 2) FDMS_PREFILL_GQA(64, 2, 4); else FDMS_PREFILL_GQA(64, 4, 4);
-    } else if (head_dim == 64) {
-      if (group == 1) FDMS_PREFILL_GQA(64, 1, 2); else if (group == 2) FDMS_PREFILL_GQA(64, 2, 2); else FDMS_PREFILL_GQA(64, 4, 2);
-    } else {
-      if (group == 1) FDMS_PREFILL_GQA(128, 1, 2); else if (group == 2) FDMS_PREFILL_GQA(128, 2, 2); else FDMS_PREFILL_GQA(128, 4, 2);
-    }
-#undef FDMS_PREFILL_GQA
-    FDMS_LAUNCH_CHECK();
-    return 0;
-  }
-  const dim3 grid((max_seqlen_q + kQRows - 1) / kQRows, num_q_heads, num_seqs);
+  const int packed = group == 2 || group == 4 ? group : 1;  // query heads per workgroup
+  const int pos = 4 * kWaveRows / packed;                   // query positions per workgroup
+  const int vec_out = ((uintptr_t)out % 16) == 0 && os_t % 8 == 0 && os_h % 8 == 0;
+  const dim3 grid((unsigned)((max_seqlen_q + pos - 1) / pos), (unsigned)(num_q_heads / packed), (unsigned)num_seqs);
+#define FDMS_PREFILL(DD, GG)                                                                                       \
+  hipLaunchKernelGGL((prefill_attn_kernel<DD, GG>), grid, dim3(kThreads), 0, (hipStream_t)stream, (const bf16_t*)q,  \
+                     qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h, (bf16_t*)out, os_t,     \
+                     os_h, cu_seqlens_q, cu_seqlens_k, group, vec_out, sl2)
   if (head_dim == 64) {
-    hipLaunchKernelGGL(prefill_attn_kernel<64>, grid, dim3(kThreads), 0, (hipStream_t)stream, (const bf16_t*)q, qs_t,
-                       qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h, (bf16_t*)out, os_t, os_h,
-                       cq, ck, group, sl2);
-  } else if (head_dim == 128) {
-    hipLaunchKernelGGL(prefill_attn_kernel<128>, grid, dim3(kThreads), 0, (hipStream_t)stream, (const bf16_t*)q,
-                       qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h, (bf16_t*)out, os_t,
-                       os_h, cq, ck, group, sl2);
+    if (packed == 1) FDMS_PREFILL(64, 1); else if (packed == 2) FDMS_PREFILL(64, 2); else FDMS_PREFILL(64, 4);
   } else {
-    return (int)hipErrorInvalidValue;
+    if (packed == 1) FDMS_PREFILL(128, 1); else if (packed == 2) FDMS_PREFILL(128, 2); else FDMS_PREFILL(128, 4);
   }
+#undef FDMS_PREFILL
   FDMS_LAUNCH_CHECK();
   return 0;
 }

@@ -264,6 +264,42 @@ def test_prefill_attention_query_tiles_agree(hq, hkv, monkeypatch):
     assert np.mean(np.abs(got - want) <= 2 ** -7 * np.abs(want) + 4e-3) > 0.99
 
 
+@pytest.mark.parametrize("d,hq,hkv,blocks,pad", [
+    (64, 8, 2, 1, 0), (64, 8, 2, 4, 8), (64, 8, 8, 5, 1), (64, 16, 2, 3, 0),
+    (128, 8, 2, 2, 1), (128, 4, 4, 3, 0), (128, 8, 4, 6, 8), (128, 8, 1, 5, 0),
+])
+def test_prefill_attention_block_edges(d, hq, hkv, blocks, pad):
+    """Lengths one below, at and above whole 64-key blocks (every parity of the
+    double-buffered pipeline, waves with fewer blocks than their workgroup,
+    the masked blocks), short chunks over a prefix, group sizes 1, 2, 4 and 8,
+    and output rows with (pad 0 / 8) and without (1) 16-byte alignment; rows
+    the call does not own keep their contents.  Tolerance: P and the output
+    rounded to bf16 (2^-9 each) against values of RMS below 1."""
+    require_gpu()
+    from fastdms_amd.layers.attention import prefill_attention
+    lens = [64 * blocks - 1, 64 * blocks, 64 * blocks + 1, 64 * blocks + 33]
+    cuts = [0, 64 * blocks - 1, 5, 64 * blocks - 31]
+    rng = np.random.default_rng(d + hq + blocks)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = int(cu[-1])
+    q, k, v = (_bf16(rng.standard_normal((t, h, d)).astype(np.float32)) for h in (hq, hkv, hkv))
+    for cut in (np.zeros(4, dtype=int), np.array(cuts)):
+        rows = np.concatenate([np.arange(cu[i] + cut[i], cu[i + 1]) for i in range(4)])
+        cq = np.concatenate([[0], np.cumsum([n - c for n, c in zip(lens, cut)])]).astype(np.int32)
+        qc = q[torch.from_numpy(rows)].contiguous()
+        want = oatt.causal_prefill_attention(qc.float().numpy(), k.float().numpy(), v.float().numpy(), cq,
+                                             cu_seqlens_k=cu)
+        buf = torch.full((len(rows) + 1, hq, d + pad), 7.0, device="cuda", dtype=torch.bfloat16)
+        out = buf[:-1, :, :d]
+        prefill_attention(qc.cuda(), k.cuda(), v.cuda(), torch.from_numpy(cq).cuda(),
+                          int(max(n - c for n, c in zip(lens, cut))), d ** -0.5, out=out,
+                          cu_seqlens_k=torch.from_numpy(cu).cuda())
+        torch.cuda.synchronize()
+        got = out.float().cpu().numpy()
+        assert np.abs(got - want).max() <= 2 ** -7 * max(1.0, np.abs(want).max())
+        assert bool((buf[-1] == 7.0).all()) and bool((buf[..., d:] == 7.0).all())
+
+
 @pytest.mark.parametrize("d,lens,cuts,hq,hkv", [
     (64, [300, 517, 64], [128, 100, 0], 8, 2),     # G = 4, prefix a multiple of 64 / not / none
     (128, [700, 129], [511, 128], 8, 2),
