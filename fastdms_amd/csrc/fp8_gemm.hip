@@ -8,18 +8,12 @@
 //   y[m, n] = bf16(y[m, n] + bias[n])                       (with a bias)
 //
 // The products of two e4m3 values are exact in fp32; the matrix cores
-// accumulate them in fp32 (v_mfma_scale_f32_16x16x128_f8f6f4 with unit E8M0
+// accumulate them in fp32 (v_mfma_scale_f32_32x32x64_f8f6f4 with unit E8M0
 // block scales), so the result differs from torch's only in summation order.
 //
-// Tiling: a workgroup computes a 128 x 128 tile of y with 4 waves of 64 x 64
-// (4 x 4 MFMA tiles of 16 x 16 each, K = 128 per instruction).  Operands go
-// straight from global memory into registers in the MFMA layout (lane group
-// g of lane (g, c) holds bytes 32 g .. 32 g + 31 of a 128-byte k-block of row
-// c), double-buffered: the next k-block is in flight while the current one
-// multiplies.  Tiles are assigned XCD by XCD (block ids are dispatched round
-// robin over the 8 XCDs), each XCD taking a contiguous run of tiles with n
-// fastest, so an x row block is read into one XCD's L2 and reused there.
-#include <cstdlib>
+// Tiles are assigned XCD by XCD (block ids are dispatched round robin over the
+// 8 XCDs), each XCD taking a contiguous run of tiles.
+#include <type_traits>
 
 #include "fdms_common.h"
 
@@ -27,279 +21,232 @@ using namespace fdms;
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kThreads = 256;
-constexpr int kBM = 128, kBN = 128, kBK = 128;
 constexpr int kGemmXcds = 8;
 
-struct Frag {
-  uint4 w[4][2];  // four 16-row weight tiles: 32 bytes of this lane's row
-  uint4 x[4][2];  // four 16-row activation tiles
-};
+// Two fp32 -> bf16 (round to nearest even) in one v_cvt_pk_bf16_f32.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t r = {(__bf16)a, (__bf16)b};
+  return __builtin_bit_cast(uint32_t, r);
+}
 
 __device__ __forceinline__ i32x8 as_i32x8(const uint4& a, const uint4& b) {
   return i32x8{(int)a.x, (int)a.y, (int)a.z, (int)a.w, (int)b.x, (int)b.y, (int)b.z, (int)b.w};
 }
 
-// Bytes k .. k + 31 of each of the lane's rows (k = block start + 32 g).
-// TAIL: the last, partial k-block; 16-byte chunks at or past K read as zero
-// (their addresses are clamped to chunk 0, in bounds).
-template <bool TAIL>
-__device__ __forceinline__ void load_frag(Frag& f, const uint8_t* const* wp, const uint8_t* const* xp, int k,
-                                          int K) {
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
-    const int kk = k + 16 * hh;
-    const bool ok = !TAIL || kk < K;
-    const int ka = ok ? kk : 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint4 vw = *reinterpret_cast<const uint4*>(wp[i] + ka);
-      const uint4 vx = *reinterpret_cast<const uint4*>(xp[i] + ka);
-      f.w[i][hh] = ok ? vw : uint4{0u, 0u, 0u, 0u};
-      f.x[i][hh] = ok ? vx : uint4{0u, 0u, 0u, 0u};
-    }
-  }
-}
-
-__device__ __forceinline__ void mma(f32x4 (&acc)[4][4], const Frag& f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const i32x8 a = as_i32x8(f.w[i][0], f.w[i][1]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, as_i32x8(f.x[j][0], f.x[j][1]), acc[i][j], 0,
-                                                                   0, 0, 127, 0, 127);
-  }
-}
-
 }  // namespace
 
-template <bool BIAS, bool VEC_OUT>
-__global__ __launch_bounds__(kThreads) void fp8_gemm_kernel(
-    const uint8_t* __restrict__ x, int64_t x_s, const float* __restrict__ x_inv, const uint8_t* __restrict__ w,
-    int64_t w_s, const float* __restrict__ w_inv, const bf16_t* __restrict__ bias, bf16_t* __restrict__ y,
-    int64_t y_s, int M, int N, int K, int tiles_n, int total, int per_xcd) {
-  const int lin = blockIdx.x;
-  const int t = (lin % kGemmXcds) * per_xcd + lin / kGemmXcds;
-  if (t >= total) return;  // uniform per workgroup
-  const int tm = t / tiles_n, tn = t - (t / tiles_n) * tiles_n;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int g = lane >> 4, c = lane & 15;
-  const int m0 = tm * kBM + (wave >> 1) * 64;
-  const int n0 = tn * kBN + (wave & 1) * 64;
-  // rows past M / N are read from the last row (in bounds) and never stored
-  const uint8_t* wp[4];
-  const uint8_t* xp[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    wp[i] = w + (int64_t)min(n0 + 16 * i + c, N - 1) * w_s;
-    xp[i] = x + (int64_t)min(m0 + 16 * i + c, M - 1) * x_s;
-  }
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int kfull = K & ~(kBK - 1);
-  const int kl = 32 * g;
-  Frag fa, fb;
-  if (kfull > 0) load_frag<false>(fa, wp, xp, kl, K);
-  for (int k0 = 0; k0 < kfull; k0 += 2 * kBK) {  // two buffers, no register copies
-    if (k0 + kBK < kfull) load_frag<false>(fb, wp, xp, k0 + kBK + kl, K);
-    mma(acc, fa);
-    if (k0 + kBK >= kfull) break;
-    if (k0 + 2 * kBK < kfull) load_frag<false>(fa, wp, xp, k0 + 2 * kBK + kl, K);
-    mma(acc, fb);
-  }
-  if (kfull < K) {
-    load_frag<true>(fa, wp, xp, kfull + kl, K);
-    mma(acc, fa);
-  }
-
-  // lane (g, c) holds C[n = n0 + 16 i + 4 g + r][m = m0 + 16 j + c]
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int m = m0 + 16 * j + c;
-    if (m >= M) continue;
-    const float xs = x_inv[m];
-    bf16_t* yr = y + (int64_t)m * y_s;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int nb = n0 + 16 * i + 4 * g;
-      if (nb >= N) continue;
-      uint32_t o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = min(nb + r, N - 1);
-        float v = acc[i][j][r] * xs * w_inv[n];
-        if (BIAS) v = bf16_to_f32(f32_to_bf16(v)) + bf16_to_f32(bias[n].bits);
-        o[r] = f32_to_bf16(v);
-      }
-      if (VEC_OUT && nb + 3 < N) {
-        *reinterpret_cast<uint2*>(yr + nb) = uint2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (nb + r < N) yr[nb + r].bits = (uint16_t)o[r];
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Large problems: 256 x 256 workgroup tiles, 4 waves of 128 x 128 (8 x 8 MFMA
-// tiles, the accumulators in AGPRs), operands staged through LDS.  Each
-// k-block (128 bytes of 256 x rows and 256 w rows, 64 KiB) is loaded by all
-// 256 threads with coalesced 16-byte loads (8 threads per row), written to
-// one of two LDS buffers, and read back by the waves in the MFMA layout; the
-// global loads of block t + 2 are in flight while block t multiplies.  LDS
-// rows are 128 bytes with the 16-byte chunks XOR-swizzled by row (chunk q of
-// row r at slot q ^ (r & 7)), so the 16 rows a fragment read touches spread
-// over the banks.
-// ---------------------------------------------------------------------------
+// Workgroup tiles of (32 TM WM) x rows by (32 TN WN) w rows on
+// v_mfma_scale_f32_32x32x64_f8f6f4 (lane l holds bytes 32 (l / 32) .. + 31 of row
+// l % 32 of a 64-byte k-step), WM x WN waves of TM x TN tiles.  k runs in stages
+// of 64 bytes per row, loaded straight into one of NS LDS buffers
+// (global_load_lds_dwordx4: no staging registers), so NS - 1 stages are in
+// flight while one multiplies.  Iteration t multiplies the fragments of stage t
+// from registers beside the LDS reads of stage t + 1; its one barrier says both
+// that stage t + 1 has landed and that stage t's buffer has been read.
+// LDS rows are 64 bytes with the 16-byte chunks XOR-swizzled (chunk q of row r
+// at slot q ^ ((r / 4) & 3)), so the 16 rows a fragment read touches at a time
+// spread over the banks.
+//
+// What bounds it: the latency of a stage's loads while few workgroups run, the
+// matrix cores and the LDS reads (96 of 128 bytes a cycle at the 256 x 256
+// tile) once the chip is full; at K = 2048 a tile's prologue and epilogue are
+// about a sixth of its time.  Measured with the row quantisation in front
+// (M x N x K, against register-staged 256 x 256 tiles of four waves with one
+// k-block in flight): 12000 x 16384 x 2048 1 033 -> 444 us (1.86 PFLOP/s), 8192 x
+// 24576 x 4096 1 615 -> 816 us, 12000 x 2048 x 2048 180 -> 79 us, 1500 x 4096 x 4096
+// 140 -> 43 us, 64 x 2048 x 8192 104 -> 29 us.
 namespace {
-constexpr int kBT = 256;      // workgroup tile, rows of x and of w
-constexpr int kRowBytes = 128;  // one k-block of a row
+constexpr int kStage = 64;  // bytes of a row per stage
+constexpr int kGroupM = 4;  // x tiles that share a run of w tiles (4 x 8 tiles per XCD at a time)
 
-struct Staging {
-  uint4 x[8];
-  uint4 w[8];
-};
-
-__device__ __forceinline__ int swz(int row, int chunk) { return row * kRowBytes + ((chunk ^ (row & 7)) << 4); }
-
-// FASTDMS_AMD_FP8_GEMM_BIG=0 keeps every problem on the 128 x 128 kernel
-bool big_tiles_enabled() {
-  static const bool on = [] {
-    const char* e = std::getenv("FASTDMS_AMD_FP8_GEMM_BIG");
-    return !(e && e[0] == '0');
-  }();
-  return on;
+// 16 bytes per lane straight into LDS at lds + 16 * lane (lds wave-uniform), from
+// a wave-uniform base + 32-bit lane offset, or from a lane's own address.  The
+// compiler does not count them: lds_dma_barrier() waits for them.
+__device__ __forceinline__ void lds_dma16(const uint8_t* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void lds_dma16_wide(const uint8_t* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
+}
+// At most N of this wave's LDS-DMA loads are still in flight and every LDS read
+// of it has returned, then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void lds_dma_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 }  // namespace
 
-template <bool BIAS, bool VEC_OUT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void fp8_gemm_big_kernel(
+template <bool BIAS, bool VEC_OUT, bool WIDE, int WM, int WN, int TM, int TN, int NS>
+__global__ __launch_bounds__(WM * WN * 64, 2) void fp8_gemm_tile_kernel(
     const uint8_t* __restrict__ x, int64_t x_s, const float* __restrict__ x_inv, const uint8_t* __restrict__ w,
     int64_t w_s, const float* __restrict__ w_inv, const bf16_t* __restrict__ bias, bf16_t* __restrict__ y,
-    int64_t y_s, int M, int N, int K, int tiles_n, int total, int per_xcd) {
-  __shared__ __attribute__((aligned(16))) uint8_t s_x[2][kBT * kRowBytes];
-  __shared__ __attribute__((aligned(16))) uint8_t s_w[2][kBT * kRowBytes];
+    int64_t y_s, int M, int N, int K, int tiles_m, int tiles_n, int total, int per_xcd) {
+  constexpr int NW = WM * WN;
+  constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
+  constexpr int XB = BM * kStage, WB = BN * kStage;  // bytes of a stage of x / w
+  constexpr int NX = XB / (1024 * NW), NWI = WB / (1024 * NW);  // LDS-DMA instructions per wave and stage
+  static_assert(NX * 1024 * NW == XB && NWI * 1024 * NW == WB, "whole LDS-DMA instructions per wave");
+  constexpr int PER = NX + NWI;
+  __shared__ __attribute__((aligned(1024))) uint8_t s_buf[NS * (XB + WB)];
+
   const int lin = blockIdx.x;
   const int t = (lin % kGemmXcds) * per_xcd + lin / kGemmXcds;
   if (t >= total) return;  // uniform per workgroup
-  const int tm = t / tiles_n, tn = t - (t / tiles_n) * tiles_n;
+  const int grp = t / (kGroupM * tiles_n), rem = t - grp * kGroupM * tiles_n;
+  const int gm = min(kGroupM, tiles_m - grp * kGroupM);  // the last group may hold fewer x tiles
+  const int tn = rem / gm, tm = grp * kGroupM + rem - tn * gm;
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int g = lane >> 4, c = lane & 15;
-  const int mb = tm * kBT, nb0 = tn * kBT;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int lc = lane & 31, half = lane >> 5;
+  const int mb = tm * BM, nb0 = tn * BN;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)s_buf;
 
-  // staging: element u of this thread is row (tid + 256 u) / 8, chunk tid % 8
-  const int srow0 = tid >> 3, schunk = tid & 7;
-  const uint8_t* xs_row[8];
-  const uint8_t* ws_row[8];
+  // LDS-DMA: instruction i of this wave moves rows 16 (i NW + wave) .. + 15 of
+  // the stage, lane l slot l % 4 of row l / 4; rows past M / N repeat the last
+  const int drow = lane >> 2, dchunk = (lane & 3) ^ ((lane >> 4) & 3);
+  using Off = typename std::conditional<WIDE, int64_t, uint32_t>::type;
+  Off xoff[NX], woff[NWI];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    xs_row[u] = x + (int64_t)min(mb + srow0 + 32 * u, M - 1) * x_s;
-    ws_row[u] = w + (int64_t)min(nb0 + srow0 + 32 * u, N - 1) * w_s;
+  for (int i = 0; i < NX; ++i) xoff[i] = (Off)min(16 * (i * NW + wave) + drow, M - 1 - mb) * (Off)x_s;
+#pragma unroll
+  for (int i = 0; i < NWI; ++i) woff[i] = (Off)min(16 * (i * NW + wave) + drow, N - 1 - nb0) * (Off)w_s;
+  const uint8_t* xb = x + (int64_t)mb * x_s;
+  const uint8_t* wb = w + (int64_t)nb0 * w_s;
+  const int nst = (K + kStage - 1) / kStage;
+  auto load_stage = [&](int st) {
+    const uint32_t buf = lds0 + (uint32_t)(st % NS) * (XB + WB);
+    const int k0 = st * kStage;
+    // the last stage's chunks past K read chunk 0 of their row (in bounds)
+    const uint32_t ko = k0 + 16 * dchunk < K ? (uint32_t)(k0 + 16 * dchunk) : 0u;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const uint32_t dst = buf + (uint32_t)((i * NW + wave) * 1024);
+      if constexpr (WIDE) lds_dma16_wide(xb + xoff[i] + ko, dst); else lds_dma16(xb, xoff[i] + ko, dst);
+    }
+#pragma unroll
+    for (int i = 0; i < NWI; ++i) {
+      const uint32_t dst = buf + XB + (uint32_t)((i * NW + wave) * 1024);
+      if constexpr (WIDE) lds_dma16_wide(wb + woff[i] + ko, dst); else lds_dma16(wb, woff[i] + ko, dst);
+    }
+  };
+
+  // fragments: lane (half, lc) holds bytes 32 half .. + 31 of row lc of a 32-row tile
+  const int xr0 = (wave / WN) * 32 * TM, wr0 = (wave % WN) * 32 * TN;
+  const int f = (lc >> 2) & 3;
+  const uint32_t a0 = lc * kStage + (((2 * half) ^ f) << 4), a1 = lc * kStage + (((2 * half + 1) ^ f) << 4);
+  struct Frags {
+    i32x8 x[TM], w[TN];
+  };
+  auto read_frags = [&](Frags& fr, int st) {
+    const uint8_t* xs = s_buf + (st % NS) * (XB + WB) + xr0 * kStage;
+    const uint8_t* ws = s_buf + (st % NS) * (XB + WB) + XB + wr0 * kStage;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+      fr.w[i] = as_i32x8(*reinterpret_cast<const uint4*>(ws + i * 32 * kStage + a0),
+                         *reinterpret_cast<const uint4*>(ws + i * 32 * kStage + a1));
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      fr.x[j] = as_i32x8(*reinterpret_cast<const uint4*>(xs + j * 32 * kStage + a0),
+                         *reinterpret_cast<const uint4*>(xs + j * 32 * kStage + a1));
+  };
+  // a partial last stage: the 16-byte chunks past K become zero in LDS
+  auto landed = [&](int st) {
+    if (K % kStage == 0 || st != nst - 1) return;  // uniform
+    uint8_t* buf = s_buf + (st % NS) * (XB + WB);
+    for (int u = tid; u < (BM + BN) * 4; u += NW * 64)
+      if (st * kStage + 16 * ((u & 3) ^ ((u >> 4) & 3)) >= K) *reinterpret_cast<uint4*>(buf + 16 * u) = uint4{0u, 0u, 0u, 0u};
+    lds_dma_barrier<0>();
+  };
+  f32x16 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x16{};
+  auto mma = [&](const Frags& fr) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fr.w[i], fr.x[j], acc[i][j], 0, 0, 0, 127, 0, 127);
+  };
+
+#pragma unroll
+  for (int st = 0; st < NS; ++st)
+    if (st < nst) load_stage(st);
+  // stage 0 has landed (fewer stages in flight than NS - 1: all have)
+  if (nst >= NS) lds_dma_barrier<(NS - 1) * PER>(); else lds_dma_barrier<0>();
+  Frags fa, fb;
+  landed(0);
+  read_frags(fa, 0);
+  // multiplies stage st (fragments cur) while stage st + 1's fragments are read
+  // into nxt: the reads are issued before the products, which hide them
+  auto step = [&](int st, Frags& cur, Frags& nxt) {
+    if (st + NS - 1 < nst) lds_dma_barrier<(NS - 2) * PER>(); else lds_dma_barrier<0>();
+    if (st + NS < nst) load_stage(st + NS);
+    landed(st + 1);
+    read_frags(nxt, st + 1);  // past the last stage: bytes no one uses
+    __builtin_amdgcn_sched_barrier(0);
+    mma(cur);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int st = 0;
+  for (; st + 1 < nst; st += 2) {
+    step(st, fa, fb);
+    step(st + 1, fb, fa);
   }
-  auto load_stage = [&](Staging& st, int blk) {
-    const int kk = blk * kRowBytes + schunk * 16;
-    const bool ok = kk < K;
-    const int ka = ok ? kk : 0;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const uint4 vx = *reinterpret_cast<const uint4*>(xs_row[u] + ka);
-      const uint4 vw = *reinterpret_cast<const uint4*>(ws_row[u] + ka);
-      st.x[u] = ok ? vx : uint4{0u, 0u, 0u, 0u};
-      st.w[u] = ok ? vw : uint4{0u, 0u, 0u, 0u};
-    }
-  };
-  auto store_stage = [&](const Staging& st, int buf) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int r = srow0 + 32 * u;
-      *reinterpret_cast<uint4*>(&s_x[buf][swz(r, schunk)]) = st.x[u];
-      *reinterpret_cast<uint4*>(&s_w[buf][swz(r, schunk)]) = st.w[u];
-    }
-  };
+  if (st < nst) step(st, fa, fb);
 
-  // wave (wy, wx): x rows wy * 128 .. + 127, w rows wx * 128 .. + 127 of the tile
-  const int xr0 = (wave >> 1) * 128, wr0 = (wave & 1) * 128;
-  f32x4 acc[8][8];
+  // lane (lc, half) holds C[n = wr0 + 32 i + 8 (r / 4) + 4 half + r % 4][m = xr0 + 32 j + lc]
+  __builtin_amdgcn_sched_barrier(0);  // the scales are not worth registers during the products
+  float xsc[TM];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int j = 0; j < TM; ++j) xsc[j] = x_inv[min(mb + xr0 + 32 * j + lc, M - 1)];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto compute = [&](int buf) {
-    i32x8 xf[8];
+  for (int i = 0; i < TN; ++i) {
+    const int nt = nb0 + wr0 + 32 * i;
+    float wsc[16], bs[16];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int r = xr0 + 16 * j + c;
-      const uint4 lo = *reinterpret_cast<const uint4*>(&s_x[buf][swz(r, 2 * g)]);
-      const uint4 hi = *reinterpret_cast<const uint4*>(&s_x[buf][swz(r, 2 * g + 1)]);
-      xf[j] = as_i32x8(lo, hi);
+    for (int r = 0; r < 16; ++r) {
+      const int n = min(nt + 8 * (r / 4) + 4 * half + r % 4, N - 1);
+      wsc[r] = w_inv[n];
+      bs[r] = BIAS ? bf16_to_f32(bias[n].bits) : 0.0f;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = wr0 + 16 * i + c;
-      const uint4 lo = *reinterpret_cast<const uint4*>(&s_w[buf][swz(r, 2 * g)]);
-      const uint4 hi = *reinterpret_cast<const uint4*>(&s_w[buf][swz(r, 2 * g + 1)]);
-      const i32x8 wf = as_i32x8(lo, hi);
+    for (int j = 0; j < TM; ++j) {
+      const int m = mb + xr0 + 32 * j + lc;
+      bf16_t* yr = y + (int64_t)min(m, M - 1) * y_s;
+      uint32_t o[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[j], acc[i][j], 0, 0, 0, 127, 0, 127);
-    }
-  };
-
-  const int nblk = (K + kRowBytes - 1) / kRowBytes;
-  Staging st;
-  load_stage(st, 0);
-  store_stage(st, 0);
-  __syncthreads();
-  if (nblk > 1) load_stage(st, 1);
-  for (int b = 0; b < nblk; ++b) {
-    compute(b & 1);
-    if (b + 1 < nblk) {
-      // buffer (b + 1) & 1 was last read in iteration b - 1, before its barrier
-      store_stage(st, (b + 1) & 1);
-      if (b + 2 < nblk) load_stage(st, b + 2);
-    }
-    __syncthreads();
-  }
-
-  // lane (g, c) holds C[n = wr0 + 16 i + 4 g + r][m = xr0 + 16 j + c] of the tile
+      for (int r = 0; r < 16; r += 2) {
+        float v[2];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int m = mb + xr0 + 16 * j + c;
-    if (m >= M) continue;
-    const float xsc = x_inv[m];
-    bf16_t* yr = y + (int64_t)m * y_s;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int nb = nb0 + wr0 + 16 * i + 4 * g;
-      if (nb >= N) continue;
-      uint32_t o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = min(nb + r, N - 1);
-        float v = acc[i][j][r] * xsc * w_inv[n];
-        if (BIAS) v = bf16_to_f32(f32_to_bf16(v)) + bf16_to_f32(bias[n].bits);
-        o[r] = f32_to_bf16(v);
+        for (int e = 0; e < 2; ++e) {
+          v[e] = acc[i][j][r + e] * xsc[j] * wsc[r + e];
+          if (BIAS) v[e] = bf16_to_f32(f32_to_bf16(v[e])) + bs[r + e];
+        }
+        o[r / 2] = pack_bf16(v[0], v[1]);
       }
-      if (VEC_OUT && nb + 3 < N) {
-        *reinterpret_cast<uint2*>(yr + nb) = uint2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
-      } else {
+      if (VEC_OUT && nt + 32 <= N) {  // uniform: the halves swap quads so that a lane stores 8 columns at once
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (nb + r < N) yr[nb + r].bits = (uint16_t)o[r];
+        for (int q = 0; q < 2; ++q) {
+          const auto s0 = __builtin_amdgcn_permlane32_swap(o[4 * q], o[4 * q + 2], false, false);
+          const auto s1 = __builtin_amdgcn_permlane32_swap(o[4 * q + 1], o[4 * q + 3], false, false);
+          if (m < M) *reinterpret_cast<uint4*>(yr + nt + 16 * q + 8 * half) = uint4{s0[0], s1[0], s0[1], s1[1]};
+        }
+      } else if (m < M) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int n = nt + 8 * (r / 4) + 4 * half + r % 4;
+          if (n < N) yr[n].bits = (uint16_t)(o[r / 2] >> (16 * (r & 1)));
+        }
       }
     }
+    if (BIAS) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -315,42 +262,39 @@ FDMS_EXPORT int fdms_fp8_gemm(const void* x, int64_t x_s, const float* x_inv, co
   if (M == 0) return 0;
   if (!x || !x_inv || !w || !w_inv || !y) return (int)hipErrorInvalidValue;
   if (((uintptr_t)x | (uintptr_t)w) & 15) return (int)hipErrorInvalidValue;
-  const bool vec = (y_s % 4) == 0 && ((uintptr_t)y % 8) == 0;
-  // 256 x 256 tiles when they fill the chip
-  const int64_t big_m = (M + kBT - 1) / kBT, big_n = (N + kBT - 1) / kBT;
-  if (big_m * big_n >= 256 && big_tiles_enabled()) {
-    const int64_t total = big_m * big_n;
-    if (total > (int64_t)0x7FFFFFFF - kGemmXcds) return (int)hipErrorInvalidValue;
-    const int per_xcd = (int)((total + kGemmXcds - 1) / kGemmXcds);
-    const dim3 grid((unsigned)(per_xcd * kGemmXcds));
-#define FDMS_GEMM_BIG(B, V)                                                                                       \
-  hipLaunchKernelGGL((fp8_gemm_big_kernel<B, V>), grid, dim3(kThreads), 0, (hipStream_t)stream, (const uint8_t*)x, \
-                     x_s, x_inv, (const uint8_t*)w, w_s, w_inv, (const bf16_t*)bias, (bf16_t*)y, y_s, M, N, K,      \
-                     (int)big_n, (int)total, per_xcd)
-    if (bias) {
-      if (vec) FDMS_GEMM_BIG(true, true); else FDMS_GEMM_BIG(true, false);
-    } else {
-      if (vec) FDMS_GEMM_BIG(false, true); else FDMS_GEMM_BIG(false, false);
-    }
-#undef FDMS_GEMM_BIG
-    FDMS_LAUNCH_CHECK();
-    return 0;
+  const bool vec = (y_s % 8) == 0 && ((uintptr_t)y % 16) == 0;
+#define FDMS_GEMM_TILE(B, V, ...)                                                                                  \
+  hipLaunchKernelGGL((fp8_gemm_tile_kernel<B, V, __VA_ARGS__>), grid, dim3(threads), 0, (hipStream_t)stream,        \
+                     (const uint8_t*)x, x_s, x_inv, (const uint8_t*)w, w_s, w_inv, (const bf16_t*)bias, (bf16_t*)y,  \
+                     y_s, M, N, K, (int)tm, (int)tn, (int)total, per_xcd)
+#define FDMS_GEMM_TILES(THREADS, BM, BN, ...)                                                                     \
+  {                                                                                                                \
+    constexpr int threads = THREADS;                                                                               \
+    const int64_t tm = tiles(M, BM), tn = tiles(N, BN), total = tm * tn;                                           \
+    if (total > (int64_t)0x7FFFFFFF - kGemmXcds) return (int)hipErrorInvalidValue;                                 \
+    const int per_xcd = (int)((total + kGemmXcds - 1) / kGemmXcds);                                                \
+    const dim3 grid((unsigned)(per_xcd * kGemmXcds));                                                              \
+    if (bias) {                                                                                                    \
+      if (vec) FDMS_GEMM_TILE(true, true, __VA_ARGS__); else FDMS_GEMM_TILE(true, false, __VA_ARGS__);             \
+    } else {                                                                                                       \
+      if (vec) FDMS_GEMM_TILE(false, true, __VA_ARGS__); else FDMS_GEMM_TILE(false, false, __VA_ARGS__);           \
+    }                                                                                                              \
+    FDMS_LAUNCH_CHECK();                                                                                           \
+    return 0;                                                                                                      \
   }
-  const int tiles_m = (M + kBM - 1) / kBM, tiles_n = (N + kBN - 1) / kBN;
-  const int64_t total = (int64_t)tiles_m * tiles_n;
-  if (total > (int64_t)0x7FFFFFFF - kGemmXcds) return (int)hipErrorInvalidValue;
-  const int per_xcd = (int)((total + kGemmXcds - 1) / kGemmXcds);
-  const dim3 grid((unsigned)(per_xcd * kGemmXcds));
-#define FDMS_GEMM_LAUNCH(B, V)                                                                                    \
-  hipLaunchKernelGGL((fp8_gemm_kernel<B, V>), grid, dim3(kThreads), 0, (hipStream_t)stream, (const uint8_t*)x, x_s, \
-                     x_inv, (const uint8_t*)w, w_s, w_inv, (const bf16_t*)bias, (bf16_t*)y, y_s, M, N, K, tiles_n,  \
-                     (int)total, per_xcd)
-  if (bias) {
-    if (vec) FDMS_GEMM_LAUNCH(true, true); else FDMS_GEMM_LAUNCH(true, false);
-  } else {
-    if (vec) FDMS_GEMM_LAUNCH(false, true); else FDMS_GEMM_LAUNCH(false, false);
-  }
-#undef FDMS_GEMM_LAUNCH
-  FDMS_LAUNCH_CHECK();
-  return 0;
+  const auto tiles = [](int n, int b) { return ((int64_t)n + b - 1) / b; };
+  // row offsets inside a tile are 32-bit below a row stride of 16 MiB
+  if (x_s >= (1 << 24) || w_s >= (1 << 24)) FDMS_GEMM_TILES(256, 64, 64, true, 2, 2, 1, 1, 6)
+  // 256 x 256 tiles (one workgroup per CU) when they fill their last round of
+  // the 256 CUs to four fifths on average: 4096^3 74 us against 92 for 128 x 128
+  // tiles (two workgroups per CU), but 5000 x 4096 x 4096 (320 tiles) 125 against
+  // 113 and 12000 x 2048 x 2048 (376 tiles) 81 against 79
+  const int64_t big = tiles(M, 256) * tiles(N, 256), rounds = (big + 255) / 256;
+  if (5 * big >= 4 * 256 * rounds) FDMS_GEMM_TILES(512, 256, 256, false, 4, 2, 2, 4, 5)
+  // 64 x 64 tiles (six stages) while 128 x 128 ones leave half the chip idle:
+  // 300 x 2048 x 8192 (48 tiles) 31 us against 46, 500 x 6144 x 4096 (192) 32 against 28
+  if (tiles(M, 128) * tiles(N, 128) >= 128) FDMS_GEMM_TILES(256, 128, 128, false, 2, 2, 2, 2, 4)
+  FDMS_GEMM_TILES(256, 64, 64, false, 2, 2, 1, 1, 6)
+#undef FDMS_GEMM_TILES
+#undef FDMS_GEMM_TILE
 }

