@@ -344,8 +344,8 @@ __global__ __launch_bounds__(NW * 64) void linear_small_m_kernel(
 #pragma unroll
           for (int a = 0; a < NA; ++a) {
             b.w4[a][u] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(wrow[a]) + kl / 2);
-            // group kl / group of weight row n: consecutive lanes read consecutive rows
-            b.gsz[a][u] = g_sz[(int64_t)(kl / group) * g_s + (n0 + c + (a ? n_out : 0))];
+            // the group of column kl of weight row n: consecutive lanes read consecutive rows
+            b.gsz[a][u] = g_sz[(int64_t)(kl >> group) * g_s + (n0 + c + (a ? n_out : 0))];
           }
         }
       }
@@ -426,37 +426,37 @@ __global__ __launch_bounds__(NW * 64) void linear_small_m_kernel(
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (kb0 + u * KB >= kend) break;
-        const bool xv = kb0 + u * KB + 32 * g < kend && has_row;  // this lane group's columns and row exist
-        // the activation operands, zeroed where they do not exist, shared by both strips
+        // the activation operands, shared by both strips (rows past M hold row
+        // 0's, whose results no one stores); a last half block's lane groups 2
+        // and 3 have no columns
         uint4 bxs[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bxs[j] = xv ? b.x8[u][j] : uint4{0u, 0u, 0u, 0u};
+        for (int j = 0; j < 4; ++j) bxs[j] = b.x8[u][j];
+        if (kb0 + u * KB + KB > kend && g >= 2) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bxs[j] = uint4{0u, 0u, 0u, 0u};
+        }
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
           // w = bf16((q - 8) * s + z) as one fma of the code: q * s + (z - 8s)
-          // (z - 8s exact for the symmetric zero 0); each byte of the masked
-          // word converts in one v_cvt_f32_ubyte, the high nibbles as 16q
-          // (with s / 16)
+          // (z - 8s exact for the symmetric zero 0).  A byte 0x0q read as e4m3fn
+          // is q * 2^-9 for every code (subnormal below 8), so one
+          // v_cvt_pk_f32_fp8 converts two codes, exactly (19 vector instructions
+          // per eight weights; with one v_cvt_f32_ubyte per code 22, and the
+          // group index by a division: gate_up of the 8B shape at four rows
+          // 21.0 -> 20.0 us, bound by the issue and latency of its loads)
           const float sc = bf_lo(b.gsz[a][u]), zc = bf_hi(b.gsz[a][u]);
-          const float c8 = __builtin_fmaf(-8.0f, sc, zc), s16 = sc * 0.0625f;
+          const float c8 = __builtin_fmaf(-8.0f, sc, zc), s9 = sc * 512.0f;
           const uint32_t wd[4] = {b.w4[a][u].x, b.w4[a][u].y, b.w4[a][u].z, b.w4[a][u].w};
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            uint32_t lo = wd[j] & 0x0F0F0F0Fu, hi = wd[j] & 0xF0F0F0F0u;
-            // hide the masks' known zero bits from the compiler: it would
-            // otherwise narrow (lo >> 8i) & 0xFF to a 4-bit field extract
-            // plus a byte-0 conversion, two instructions instead of one
-            // v_cvt_f32_ubyte<i> per code
-            asm("" : "+v"(lo), "+v"(hi));
-            const uint4 aw = uint4{
-                pack2(__builtin_fmaf((float)(lo & 0xFFu), sc, c8),
-                      __builtin_fmaf((float)(hi & 0xFFu), s16, c8)),
-                pack2(__builtin_fmaf((float)((lo >> 8) & 0xFFu), sc, c8),
-                      __builtin_fmaf((float)((hi >> 8) & 0xFFu), s16, c8)),
-                pack2(__builtin_fmaf((float)((lo >> 16) & 0xFFu), sc, c8),
-                      __builtin_fmaf((float)((hi >> 16) & 0xFFu), s16, c8)),
-                pack2(__builtin_fmaf((float)((lo >> 24) & 0xFFu), sc, c8),
-                      __builtin_fmaf((float)((hi >> 24) & 0xFFu), s16, c8))};
+            const int lo = (int)(wd[j] & 0x0F0F0F0Fu), hi = (int)((wd[j] >> 4) & 0x0F0F0F0Fu);
+            const auto l0 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), l1 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, true);
+            const auto h0 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, false), h1 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, true);
+            const uint4 aw = uint4{pack2(__builtin_fmaf(l0[0], s9, c8), __builtin_fmaf(h0[0], s9, c8)),
+                                   pack2(__builtin_fmaf(l0[1], s9, c8), __builtin_fmaf(h0[1], s9, c8)),
+                                   pack2(__builtin_fmaf(l1[0], s9, c8), __builtin_fmaf(h1[0], s9, c8)),
+                                   pack2(__builtin_fmaf(l1[1], s9, c8), __builtin_fmaf(h1[1], s9, c8))};
             acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(aw), as_bf16x8(bxs[j]), acc[a], 0, 0, 0);
           }
         }
@@ -938,7 +938,7 @@ struct LinArgs {
   const bf16_t* x; int64_t x_s; int M, K; const void* w; int64_t w_s; const float* wsi; const bf16_t* bias;
   const bf16_t* norm_w; float eps; const bf16_t* res; int64_t res_s; bf16_t* res_out; int64_t ro_s;
   bf16_t* y; int64_t y_s; int n_out, strips, ksplit; float* ws; int* counters; float* pval; int* pidx;
-  const uint32_t* g_sz = nullptr; int group = 1; int64_t g_s = 0;
+  const uint32_t* g_sz = nullptr; int group = 0; int64_t g_s = 0;  // group: log2 of the group size
   int qx_torch = 0; int bf16_scores = 1;
   const float* x_amax = nullptr; int x_amax_n = 0; int64_t x_amax_s = 0; float* amax_out = nullptr;
   float* row_scale_out = nullptr;
@@ -1322,7 +1322,7 @@ FDMS_EXPORT int fdms_linear_int4_small_m(const void* x, int64_t x_stride, int m,
             nullptr, 0, nullptr, 0, (bf16_t*)y, y_stride, n_out, strips, k_splits, workspace, counters, part_val,
             part_idx};
   a.g_sz = (const uint32_t*)scale_zeros;
-  a.group = group_size;
+  a.group = __builtin_ctz((unsigned)group_size);
   a.g_s = sz_stride;
   const dim3 grid((unsigned)blocks);
   const hipStream_t st = (hipStream_t)stream;

@@ -66,16 +66,21 @@ def choose_k_splits(device: torch.device, strips: int, k: int) -> int:
     return s
 
 
-def choose_partial_splits(device: torch.device, strips: int, k: int) -> int:
+def choose_partial_splits(device: torch.device, strips: int, k: int, per_cu: int = 2) -> int:
     """K splits of a linear whose merge the consumer does (no merge cost in the
-    linear): enough workgroups to cover the CUs, each split a whole number of
-    512-column slices.  FASTDMS_AMD_PARTIAL_SPLITS overrides (tuning)."""
+    linear): up to ``per_cu`` workgroups per CU, each split a whole number of
+    512-column slices.  One workgroup per CU is one wave per SIMD, which alone
+    issues a vector instruction every eight cycles instead of four and waits
+    out each of its loads: two per CU measured 1.5 % (bf16), 2-4 % (FP8) faster
+    over a decode MLP; INT4, whose weights are converted in the vector unit,
+    takes four (13 % at hidden 4096; FP8 4 % slower there at four).
+    FASTDMS_AMD_PARTIAL_SPLITS overrides (tuning)."""
     env = os.environ.get("FASTDMS_AMD_PARTIAL_SPLITS", "").strip()
     if env.isdigit() and int(env) >= 1 and k % (int(env) * 256) == 0:
         return int(env)
     s = 1
-    cus = _num_cus(device)
-    while s * 2 <= _MAX_K_SPLITS and strips * s < cus and k % (s * 2 * 512) == 0:
+    target = per_cu * _num_cus(device)
+    while s * 2 <= _MAX_K_SPLITS and strips * s < target and k % (s * 2 * 512) == 0:
         s *= 2
     return s
 
@@ -488,7 +493,7 @@ def linear_int4_partials(x: torch.Tensor, packed: torch.Tensor, scale_zeros: tor
     if not small_m_supported(rows, k, n):
         raise ValueError(f"linear_int4_partials does not support rows={rows}, K={k}, N={n}")
     if k_splits is None:
-        k_splits = choose_partial_splits(x.device, n // 16, k)
+        k_splits = choose_partial_splits(x.device, n // 16, k, per_cu=4)
     part = _partials_buffer(x.device, k_splits, rows, n)
     nat.require_cuda(x, packed, scale_zeros, what="linear_int4_partials")
     nat.call("fdms_linear_int4_small_m", x.data_ptr(), x.stride(0), rows, k, packed.data_ptr(), packed.stride(0),

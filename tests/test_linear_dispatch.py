@@ -173,3 +173,16 @@ def test_norm_stats_buffers_must_match_the_strips():
         linear_norm_stats(f, torch.zeros(rows, n // 16 + 1), nw, 1e-5, w2, epilogue=EPI_SILU_MUL)
     with pytest.raises(ValueError, match="ssq must be"):
         linear_norm_stats(f, torch.zeros(rows, n // 32), nw, 1e-5, w2, epilogue=EPI_SILU_MUL)
+
+
+@pytest.mark.parametrize("strips,k,per_cu,want", [
+    (128, 8192, 2, 4), (128, 2048, 2, 4), (256, 12288, 2, 2), (256, 12288, 4, 4), (512, 8192, 2, 1),
+    (128, 1024, 4, 2), (16, 16384, 4, 8), (128, 1536, 2, 1)])
+def test_partial_splits_fill_the_chip_in_whole_slices(strips, k, per_cu, want, monkeypatch):
+    """choose_partial_splits doubles the K splits up to per_cu workgroups per
+    CU, at most eight, each split whole 512-column slices."""
+    from fastdms_amd.layers import linear as lin
+    monkeypatch.delenv("FASTDMS_AMD_PARTIAL_SPLITS", raising=False)
+    monkeypatch.setattr(lin, "_num_cus", lambda device: 256)
+    got = lin.choose_partial_splits(torch.device("cpu"), strips, k, per_cu=per_cu)
+    assert got == want and (got == 1 or k % (got * 512) == 0)
