@@ -98,6 +98,31 @@ def test_silu_mul(rows, f):
     _ulp_close(out, want, "silu_mul")
 
 
+@pytest.mark.parametrize("rows,f", [(3, 8), (1030, 8), (127, 24), (2047, 8192), (2048, 8192), (2049, 8200),
+                                    (700000, 24), (2100001, 8), (3, 5592408)])
+def test_silu_mul_sizes(rows, f):
+    """The last workgroup's remainder, workgroups that span many rows and the
+    two sides of the line to several units a thread (2 047 workgroups of
+    1 024 8-column units): within a bf16 step of torch's fp32 expression, NaN
+    where it is NaN, nothing written past the end."""
+    require_gpu()
+    from fastdms_amd.layers.activation import silu_and_mul
+    g = torch.Generator(device="cuda").manual_seed(rows + f)
+    x = (3 * torch.randn(rows, 2 * f, generator=g, device="cuda")).to(torch.bfloat16)
+    special = torch.tensor([float("nan"), float("inf"), -float("inf"), -90.0, 90.0, 0.0, -0.0], dtype=torch.bfloat16)
+    x[0, :7] = special.cuda()
+    x[-1, 1:8] = special.cuda()
+    buf = torch.full((rows * f + 4096,), 7.0, device="cuda", dtype=torch.bfloat16)
+    out = silu_and_mul(x, out=buf[:rows * f].view(rows, f))
+    assert bool((buf[rows * f:] == 7.0).all())
+    a, b = x[:, :f].float(), x[:, f:].float()
+    want = (a / (1.0 + torch.exp(-a)) * b).to(torch.bfloat16)
+    assert torch.equal(torch.isnan(out), torch.isnan(want))
+    o, w = torch.nan_to_num(out.float()), torch.nan_to_num(want.float())
+    # 2^-7 relative is one bf16 step: fp32 roundings of either side may cross one rounding boundary
+    assert bool(((o - w).abs() <= w.abs() * 2.0 ** -7 + 1e-36).all())
+
+
 @pytest.mark.parametrize("vocab,dim,n", [(128256, 2048, 8), (1000, 4096, 3000), (512, 264, 17)])
 def test_fp8_embedding_gather_matches_the_oracle(vocab, dim, n):
     """(f)2: the FP8 embedding gather equals the oracle's rows bit for bit
