@@ -36,6 +36,7 @@ SIGNATURES: dict[str, str] = {
     "fdms_streaming_pack_scatter": "ppillllpllpllpllplppilpllplliiiiippp",
     "fdms_dms_rope_store_compact_decode": "pillppillllpllppilpllpllpiiiifffiiippp",
     "fdms_rope_inplace": "pillliipllpp",
+    "fdms_prefill_qk": "pllipllilipfpfpllfffiplpp",
     "fdms_store_compact_kvcache": "ppillllppilplliiippp",
     "fdms_compact_decode_attention": "pillppilpllpllipllpllppiiiiiifpllpppp",
     "fdms_fused_decode_attention": "pllpllpllpllppllpllfffipplpllpllpllppiiiiiifppppfp",

@@ -396,6 +396,127 @@ FDMS_EXPORT int fdms_embedding_fp8(const int64_t* ids, int64_t n, const void* ta
   return 0;
 }
 
+// Everything a prefill attention layer does to q and k between the qkv linear
+// and the pack / attention, in place on views of the qkv rows: (Qwen3) the
+// per-head RMSNorm of q and k, the DMS decision of each kv head's first query
+// head (channel D - 1, then zeroed), RoPE of q and k -- the bits of
+// rmsnorm_rows_kernel, extract_dms_kernel and rope_inplace_kernel one after the
+// other, which read and write the rows up to three times in five launches.
+// One workgroup per token, T = D / 8 lanes per head, two heads per lane group
+// with both loads issued before the first use; a head's two halves meet
+// through a lane shuffle of the bf16 pairs.  Bound by HBM: 4 D bytes per head
+// and token, and the cos / sin row once per token.
+// 12 000 tokens of the 8B shape (32 + 8 heads of 128): the five launches 132 us,
+// this one 47 us (5.2 TB/s).
+__device__ __forceinline__ float rope_half(float x, float other, float c, float signed_s) {
+#pragma clang fp contract(off)
+  const float a = x * c, b = other * signed_s;  // rope_f32's products and sum: x1 c + x2 (-s) or x2 c + x1 s
+  return a + b;
+}
+template <int T, bool NORM>
+__global__ __launch_bounds__(1024) void prefill_qk_kernel(
+    bf16_t* __restrict__ q, int64_t qs_t, int64_t qs_h, int hq, bf16_t* __restrict__ k, int64_t ks_t, int64_t ks_h,
+    int hkv, const bf16_t* __restrict__ q_weight, float q_eps, const bf16_t* __restrict__ k_weight, float k_eps,
+    uint8_t* __restrict__ evict, int64_t es_t, int64_t es_h, float alpha_scale, float alpha_offset, float threshold,
+    int positive_scale, const float* __restrict__ cos_sin, int64_t cs_p, const int64_t* __restrict__ positions) {
+  constexpr int V = 8, P = 2, kHalf = T * V / 2;
+  const int64_t t = blockIdx.x;
+  const int groups = blockDim.x / T, lane = threadIdx.x % T, c = lane * V;
+  const int heads = hq + hkv, group = hq / hkv;
+  bf16_t* rows[P];
+  Vec<bf16_t, V> xv[P], wv[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int h = min((int)(threadIdx.x / T) + p * groups, heads - 1);
+    rows[p] = h < hq ? q + t * qs_t + h * qs_h : k + t * ks_t + (h - hq) * ks_h;
+    xv[p] = *reinterpret_cast<const Vec<bf16_t, V>*>(rows[p] + c);
+    if constexpr (NORM) wv[p] = *reinterpret_cast<const Vec<bf16_t, V>*>((h < hq ? q_weight : k_weight) + c);
+  }
+  const bool upper = c >= kHalf;
+  const float* cs = cos_sin + positions[t] * cs_p + (upper ? c - kHalf : c);
+  const Vec<float, 4> cv[2] = {*reinterpret_cast<const Vec<float, 4>*>(cs), *reinterpret_cast<const Vec<float, 4>*>(cs + 4)};
+  Vec<float, 4> sv[2] = {*reinterpret_cast<const Vec<float, 4>*>(cs + kHalf),
+                         *reinterpret_cast<const Vec<float, 4>*>(cs + kHalf + 4)};
+#pragma unroll
+  for (int i = 0; i < V; ++i) sv[i / 4].v[i % 4] = upper ? sv[i / 4].v[i % 4] : -sv[i / 4].v[i % 4];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int h = (int)(threadIdx.x / T) + p * groups;
+    const bool valid = h < heads;  // the lanes past the last head repeat it without storing
+    float x[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) x[i] = bf16_to_f32(xv[p].v[i].bits);
+    if constexpr (NORM) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int i = 0; i < V; ++i) ss += x[i] * x[i];
+      ss = segment_sum<T>(ss);
+      const float inv = rsqrtf(ss / (float)(V * T) + (h < hq ? q_eps : k_eps));
+#pragma unroll
+      for (int i = 0; i < V; i += 2) {
+        const uint32_t xn = pack_bf16(x[i] * inv, x[i + 1] * inv);
+        const uint32_t o = pack_bf16(__uint_as_float(xn << 16) * bf16_to_f32(wv[p].v[i].bits),
+                                     __uint_as_float(xn & 0xFFFF0000u) * bf16_to_f32(wv[p].v[i + 1].bits));
+        x[i] = __uint_as_float(o << 16);
+        x[i + 1] = __uint_as_float(o & 0xFFFF0000u);
+      }
+    }
+    if (valid && h < hq && h % group == 0 && lane == T - 1) {
+      evict[t * es_t + (h / group) * es_h] =
+          dms_decide(x[V - 1], alpha_scale, alpha_offset, threshold, positive_scale) ? 1 : 0;
+      x[V - 1] = 0.0f;
+    }
+    uint32_t o[V / 2];
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i) {
+      // exact: the values are bf16
+      const uint32_t mine = (__float_as_uint(x[2 * i]) >> 16) | (__float_as_uint(x[2 * i + 1]) & 0xFFFF0000u);
+      const uint32_t other = __shfl_xor(mine, T / 2);
+      float y[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float xo = __uint_as_float(e ? other & 0xFFFF0000u : other << 16);
+        y[e] = rope_half(x[2 * i + e], xo, cv[i / 2].v[(2 * i + e) % 4], sv[i / 2].v[(2 * i + e) % 4]);
+      }
+      o[i] = pack_bf16(y[0], y[1]);
+    }
+    if (valid) *reinterpret_cast<uint4*>(rows[p] + c) = uint4{o[0], o[1], o[2], o[3]};
+  }
+}
+
+// q [tokens, hq, D] and k [tokens, hkv, D] bf16 views (element strides), D 64 or
+// 128, (hq + hkv) * D / 8 <= 2048 lanes; q_weight / k_weight both [D] or both
+// NULL (no norm); evict [tokens, hkv] bytes; cos_sin fp32 rows cat(cos, sin) of D
+// values, cs_p apart.
+FDMS_EXPORT int fdms_prefill_qk(void* q, int64_t qs_t, int64_t qs_h, int hq, void* k, int64_t ks_t, int64_t ks_h,
+                                int hkv, int64_t num_tokens, int head_dim, const void* q_weight, float q_eps,
+                                const void* k_weight, float k_eps, uint8_t* evict, int64_t es_t, int64_t es_h,
+                                float alpha_scale, float alpha_offset, float threshold, int positive_scale,
+                                const float* cos_sin, int64_t cs_p, const int64_t* positions, void* stream) {
+  if (num_tokens < 0 || hkv <= 0 || hq <= 0 || hq % hkv || (head_dim != 64 && head_dim != 128))
+    return (int)hipErrorInvalidValue;
+  const int lanes = head_dim / 8;
+  if ((int64_t)(hq + hkv) * lanes > 2048 || (q_weight == nullptr) != (k_weight == nullptr)) return (int)hipErrorInvalidValue;
+  if (num_tokens == 0) return 0;
+  if (!q || !k || !evict || !cos_sin || !positions || num_tokens > 0x7FFFFFFF) return (int)hipErrorInvalidValue;
+  if (!fdms_aligned16(q, k, q_weight, k_weight, cos_sin) || (qs_t | qs_h | ks_t | ks_h) % 8 || cs_p % 4)
+    return (int)hipErrorInvalidValue;
+  const int threads = ((hq + hkv + 1) / 2 * lanes + kWave - 1) / kWave * kWave;
+#define FDMS_PREFILL_QK(TV, NV)                                                                                    \
+  hipLaunchKernelGGL((prefill_qk_kernel<TV, NV>), dim3((unsigned)num_tokens), dim3((unsigned)threads), 0,             \
+                     (hipStream_t)stream, (bf16_t*)q, qs_t, qs_h, hq, (bf16_t*)k, ks_t, ks_h, hkv,                     \
+                     (const bf16_t*)q_weight, q_eps, (const bf16_t*)k_weight, k_eps, evict, es_t, es_h, alpha_scale,   \
+                     alpha_offset, threshold, positive_scale, cos_sin, cs_p, positions)
+  if (lanes == 8) {
+    if (q_weight) FDMS_PREFILL_QK(8, true); else FDMS_PREFILL_QK(8, false);
+  } else {
+    if (q_weight) FDMS_PREFILL_QK(16, true); else FDMS_PREFILL_QK(16, false);
+  }
+#undef FDMS_PREFILL_QK
+  FDMS_LAUNCH_CHECK();
+  return 0;
+}
+
 // out[r, j] = bf16(silu(x[r, j]) * x[r, F + j]) in fp32 (activation.py:8-11).
 // A workgroup takes 256 U consecutive 8-column units of the output, a thread U
 // of them, 256 apart; all its loads (2 U of 16 bytes) go out before the first

@@ -132,6 +132,39 @@ def extract_dms_eviction_decisions(q: torch.Tensor, *, num_kv_heads: int, num_qo
     return q_clean, evict_mask
 
 
+def prefill_qk_supported(q: torch.Tensor, k: torch.Tensor, cos_sin_cache: torch.Tensor, norms: tuple = ()) -> bool:
+    """Views that fdms_prefill_qk takes: bf16 rows of 64 or 128 values moved as
+    16-byte vectors, at most 2 048 such vectors per token, fp32 cos / sin rows."""
+    d = q.shape[2]
+    tensors = (q, k, cos_sin_cache) + tuple(n.weight for n in norms)
+    return (q.dtype == k.dtype == torch.bfloat16 and d in (64, 128) and q.shape[0] > 0
+            and q.shape[1] % k.shape[1] == 0 and (q.shape[1] + k.shape[1]) * d // 8 <= 2048
+            and q.stride(2) == k.stride(2) == 1
+            and all(s % 8 == 0 for s in (q.stride(0), q.stride(1), k.stride(0), k.stride(1)))
+            and cos_sin_cache.dtype == torch.float32 and cos_sin_cache.stride(2) == 1
+            and cos_sin_cache.stride(0) % 4 == 0
+            and all(n.weight.dtype == torch.bfloat16 and n.weight.is_contiguous() for n in norms)
+            and all(t.data_ptr() % 16 == 0 for t in tensors))
+
+
+def prefill_qk_inplace(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor, cos_sin_cache: torch.Tensor, *,
+                       alpha_scale: float, alpha_offset: float, norms: tuple = ()) -> torch.Tensor:
+    """q [T, Hq, D] and k [T, Hkv, D] (prefill_qk_supported) through (norms: the
+    q and k RMSNorm modules) QK-norm, DMS decisions and RoPE, in place and in one
+    launch; returns the eviction mask [T, Hkv]."""
+    nat.require_cuda(q, k, positions, cos_sin_cache, what="prefill_qk_inplace")
+    pos = positions if positions.dtype == torch.int64 else positions.to(torch.int64)
+    evict = torch.empty((q.shape[0], k.shape[1]), device=q.device, dtype=torch.bool)
+    qn, kn = norms if norms else (None, None)
+    nat.call("fdms_prefill_qk", q.data_ptr(), q.stride(0), q.stride(1), q.shape[1], k.data_ptr(), k.stride(0),
+             k.stride(1), k.shape[1], q.shape[0], q.shape[2], qn.weight.data_ptr() if norms else None,
+             float(qn.eps) if norms else 0.0, kn.weight.data_ptr() if norms else None,
+             float(kn.eps) if norms else 0.0, evict.data_ptr(), evict.stride(0), evict.stride(1),
+             *dms_threshold_args(alpha_scale, alpha_offset), cos_sin_cache.data_ptr(), cos_sin_cache.stride(0),
+             pos.data_ptr(), nat.stream())
+    return evict
+
+
 def build_dms_live_mask(evict_mask: torch.Tensor, *, current_position: int, window_size: int,
                         positions: torch.Tensor | None = None) -> torch.Tensor:
     """dms.py:235-262: live = ~evict | (current - pos <= window)."""

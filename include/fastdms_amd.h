@@ -129,6 +129,16 @@ int fdms_rope_inplace(void* x, int dtype, int64_t xs_t, int64_t xs_h, int64_t nu
                       int head_dim, const float* cos_sin, int64_t cs_p, int64_t cs_d, const int64_t* positions,
                       void* stream);
 
+/* Prefill q / k between the qkv linear and the pack / attention, in place on
+ * bf16 views: per-head RMSNorm (both weights NULL: none), DMS decision of each
+ * kv head's first query head (channel zeroed), RoPE.  The results of
+ * fdms_rmsnorm, fdms_extract_dms_decisions and fdms_rope_inplace in turn. */
+int fdms_prefill_qk(void* q, int64_t qs_t, int64_t qs_h, int hq, void* k, int64_t ks_t, int64_t ks_h, int hkv,
+                    int64_t num_tokens, int head_dim, const void* q_weight, float q_eps, const void* k_weight,
+                    float k_eps, uint8_t* evict, int64_t es_t, int64_t es_h, float alpha_scale,
+                    float alpha_offset, float threshold, int positive_scale, const float* cos_sin, int64_t cs_p,
+                    const int64_t* positions, void* stream);
+
 /* A10 — unfused append store.  Replaces _store_compact_kvcache_kernel /
  * store_compact_kvcache (compact_attention.py:212-246, 968-1007). */
 int fdms_store_compact_kvcache(const void* key, const void* value, int kv_dtype, int64_t ks_b, int64_t ks_h,

@@ -324,6 +324,28 @@ class Emulator:
         self.store(xv, torch.cat([y1, y2], -1), dt)
         return 0
 
+    def prefill_qk(self, q, qs_t, qs_h, HQ, k, ks_t, ks_h, HKV, T, D, q_weight, q_eps, k_weight, k_eps, evict, es_t,
+                   es_h, a_s, a_o, thr, pos_scale, cos_sin, cs_p, positions, stream):
+        if HKV <= 0 or HQ % HKV or D not in (64, 128) or (HQ + HKV) * D // 8 > 2048 or bool(q_weight) != bool(k_weight):
+            return 1
+        if any(p % 16 for p in (q, k, q_weight or 0, k_weight or 0, cos_sin)) or cs_p % 4 \
+                or any(s % 8 for s in (qs_t, qs_h, ks_t, ks_h)):
+            return 1
+        for x, s_t, s_h, heads, weight, eps in ((q, qs_t, qs_h, HQ, q_weight, q_eps), (k, ks_t, ks_h, HKV, k_weight, k_eps)):
+            if weight:
+                xv = self.view(x, torch.bfloat16, (T, heads, D), (s_t, s_h, 1), "prefill_qk rows")
+                normed = torch.empty((T, heads, D), dtype=torch.bfloat16)
+                f = xv.float()
+                inv = torch.rsqrt((f * f).sum(-1, keepdim=True) / D + eps)
+                w = self.view(weight, torch.bfloat16, (D,), (1,), "weight").float()
+                normed.copy_(((f * inv).to(torch.bfloat16).float() * w).to(torch.bfloat16))
+                xv.copy_(normed)
+        bf16 = [c for c, d in _TORCH.items() if d == torch.bfloat16][0]
+        return (self.extract_dms_decisions(q, bf16, qs_t, qs_h, 1, evict, es_t, es_h, T, HKV, HQ // HKV, D, a_s, a_o,
+                                           thr, pos_scale, stream)
+                or self.rope_inplace(q, bf16, qs_t, qs_h, T, HQ, D, cos_sin, cs_p, 1, positions, stream)
+                or self.rope_inplace(k, bf16, ks_t, ks_h, T, HKV, D, cos_sin, cs_p, 1, positions, stream))
+
     def dms_rope_store_compact_decode(self, q, qdt, qs_b, qs_h, k, v, kvdt, ks_b, ks_h, vs_b, vs_h, cos_sin, cs_p,
                                       cs_d, ck, cv, cdt, c_s, slot, sm_b, sm_h, ev_out, ev_b, ev_h, positions, B, H,
                                       G, D, a_s, a_o, thr, pos_scale, store_q, store_tk, k_scale, v_scale, stream):

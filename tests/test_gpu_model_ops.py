@@ -98,6 +98,46 @@ def test_silu_mul(rows, f):
     _ulp_close(out, want, "silu_mul")
 
 
+@pytest.mark.parametrize("tokens,hq,hkv,d,norm", [(1, 1, 1, 64, False), (7, 32, 8, 64, False), (300, 32, 8, 128, True),
+                                                  (5, 3, 1, 128, True), (3, 5, 5, 64, True), (2, 112, 16, 128, False),
+                                                  (2, 128, 128, 64, True)])
+def test_prefill_qk_matches_the_separate_kernels(tokens, hq, hkv, d, norm):
+    """QK-norm, decision and RoPE in one launch give the bits of the kernels one
+    after the other; v and the neighbouring columns stay as they are.  Odd head
+    counts leave lanes without a head; 128 / 256 heads are the largest grids."""
+    require_gpu()
+    from fastdms_amd.engine.dms import extract_dms_eviction_decisions, prefill_qk_inplace, prefill_qk_supported
+    from fastdms_amd.layers.layernorm import RMSNorm, rms_norm
+    from fastdms_amd.layers.rotary_embedding import build_cos_sin_cache, rope_inplace
+    g = torch.Generator().manual_seed(tokens * hq + d)
+    qkv = torch.randn(tokens, (hq + 2 * hkv) * d, generator=g).to(torch.bfloat16).cuda()
+    want_rows = qkv.clone()
+    pos = torch.randint(0, 512, (tokens,), generator=g).cuda()
+    table = build_cos_sin_cache(d, 512, 10000.0).cuda()
+    norms = ()
+    if norm:
+        norms = tuple(RMSNorm(d, eps=e).cuda() for e in (1e-6, 1e-2))
+        for n in norms:
+            n.weight.data = (1.0 + 0.3 * torch.randn(d, generator=g)).to(torch.bfloat16).cuda()
+
+    def views(rows):
+        return (rows[:, :hq * d].view(-1, hq, d), rows[:, hq * d:(hq + hkv) * d].view(-1, hkv, d))
+
+    q, k = views(want_rows)
+    if norm:
+        q, k = (rms_norm(x, n.weight, n.eps) for x, n in zip((q, k), norms))
+    q, want_evict = extract_dms_eviction_decisions(q, num_kv_heads=hkv, num_qo_heads=hq, head_dim=d, alpha_scale=10.0,
+                                                   alpha_offset=1.0, inplace=True)
+    want_q, want_k = rope_inplace(q, pos, table), rope_inplace(k, pos, table)
+    v = qkv[:, (hq + hkv) * d:].clone()
+    q, k = views(qkv)
+    assert prefill_qk_supported(q, k, table, norms)
+    evict = prefill_qk_inplace(q, k, pos, table, alpha_scale=10.0, alpha_offset=1.0, norms=norms)
+    assert torch.equal(evict, want_evict)
+    assert torch.equal(q, want_q) and torch.equal(k, want_k)
+    assert torch.equal(qkv[:, (hq + hkv) * d:], v)
+
+
 @pytest.mark.parametrize("rows,f", [(3, 8), (1030, 8), (127, 24), (2047, 8192), (2048, 8192), (2049, 8200),
                                     (700000, 24), (2100001, 8), (3, 5592408)])
 def test_silu_mul_sizes(rows, f):
