@@ -66,14 +66,19 @@ def choose_k_splits(device: torch.device, strips: int, k: int) -> int:
     return s
 
 
-def choose_partial_splits(device: torch.device, strips: int, k: int, per_cu: int = 2) -> int:
+def choose_partial_splits(device: torch.device, strips: int, k: int, per_cu: int = 1) -> int:
     """K splits of a linear whose merge the consumer does (no merge cost in the
     linear): up to ``per_cu`` workgroups per CU, each split a whole number of
     512-column slices.  One workgroup per CU is one wave per SIMD, which alone
     issues a vector instruction every eight cycles instead of four and waits
-    out each of its loads: two per CU measured 1.5 % (bf16), 2-4 % (FP8) faster
-    over a decode MLP; INT4, whose weights are converted in the vector unit,
-    takes four (13 % at hidden 4096; FP8 4 % slower there at four).
+    out each of its loads, but more splits are more partial sums to write and
+    merge.  Over three-layer decode MLPs, against one per CU: FP8 takes two
+    (hidden 4096, 2 / 15 rows 166.5 -> 161.0 / 190.0 -> 188.4 us; 2048 72.5 ->
+    72.4 / 83.0 -> 81.3; four are 4-8 % slower); INT4, whose weights are
+    converted in the vector unit, four (4096 114.5 -> 102.1 / 148.4 -> 141.0;
+    2048 63.0 -> 60.7 / 75.2 -> 73.6); bf16 stays at one (two: 2048 88.0 ->
+    86.7 / 98.1 -> 97.8, but 4096 at 15 rows 217 -> 220 and a decode forward of
+    the 8B shape 575 -> 577).
     FASTDMS_AMD_PARTIAL_SPLITS overrides (tuning)."""
     env = os.environ.get("FASTDMS_AMD_PARTIAL_SPLITS", "").strip()
     if env.isdigit() and int(env) >= 1 and k % (int(env) * 256) == 0:
@@ -152,7 +157,7 @@ def linear_partials(x: torch.Tensor, weight: torch.Tensor, k_splits: int | None 
         raise ValueError(f"linear_partials does not support rows={rows}, K={k}, N={n}")
     am_ptr, am_n, am_s = _amax_args(x_amax if qx else None, rows)
     if k_splits is None:
-        k_splits = choose_partial_splits(x.device, n // 16, k)
+        k_splits = choose_partial_splits(x.device, n // 16, k, per_cu=2 if fp8 else 1)
     part = _partials_buffer(x.device, k_splits, rows, n)
     idx = _device_index(x.device)
     sinv = row_scale = None

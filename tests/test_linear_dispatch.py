@@ -186,3 +186,30 @@ def test_partial_splits_fill_the_chip_in_whole_slices(strips, k, per_cu, want, m
     monkeypatch.setattr(lin, "_num_cus", lambda device: 256)
     got = lin.choose_partial_splits(torch.device("cpu"), strips, k, per_cu=per_cu)
     assert got == want and (got == 1 or k % (got * 512) == 0)
+
+
+@pytest.mark.parametrize("weights,n,k,want", [
+    ("bf16", 2048, 8192, 2), ("bf16", 2048, 2048, 2), ("bf16", 4096, 12288, 1),
+    ("fp8", 2048, 8192, 4), ("fp8", 4096, 12288, 2), ("int4", 2048, 8192, 8), ("int4", 4096, 12288, 4)])
+def test_partial_splits_of_each_weight_type(weights, n, k, want, monkeypatch):
+    """One workgroup per CU for bf16 rows, whose sums keep the order (and the
+    bits) of two splits at hidden 2048 and one at 4096; two for FP8, four for
+    INT4."""
+    from fastdms_amd.layers import linear as lin
+    monkeypatch.delenv("FASTDMS_AMD_PARTIAL_SPLITS", raising=False)
+    monkeypatch.setattr(lin, "_num_cus", lambda device: 256)
+    monkeypatch.setattr(lin, "_device_index", lambda device: 0)
+    monkeypatch.setattr(lin, "_PARTIALS", {})
+    monkeypatch.setattr(lin, "_ROW_SCALES", {})
+    monkeypatch.setattr(lin.nat, "require_cuda", lambda *a, **kw: None)
+    monkeypatch.setattr(lin.nat, "stream", lambda: None)
+    monkeypatch.setattr(lin.nat, "call", lambda *a: None)
+    x = torch.zeros(8, k, dtype=torch.bfloat16)
+    if weights == "int4":
+        got = lin.linear_int4_partials(x, torch.zeros(n, k // 2, dtype=torch.uint8),
+                                       torch.zeros(k // 128, n, 2, dtype=torch.bfloat16), 128)
+    elif weights == "fp8":
+        got = lin.linear_partials(x, torch.zeros(n, k, dtype=torch.float8_e4m3fn), weight_scale_inv=torch.ones(n))
+    else:
+        got = lin.linear_partials(x, torch.zeros(n, k, dtype=torch.bfloat16))
+    assert got.data.shape == (want, 8, n)
