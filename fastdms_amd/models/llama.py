@@ -26,7 +26,7 @@ from ..layers.layernorm import RMSNorm
 from ..layers.linear import (EPI_NONE, EPI_SILU_MUL, LinearBase, MergedColumnParallelLinear, QKVParallelLinear,
                              RowParallelLinear, linear_int4_partials, linear_norm_stats, linear_partials,
                              linear_residual_stats, small_m_supported)
-from ..layers.rotary_embedding import get_rope
+from ..layers.rotary_embedding import RotaryEmbedding, get_rope
 from ..utils.context import get_context
 
 
@@ -130,6 +130,16 @@ def _norm_stats_enabled(hidden_size: int) -> bool:
     return hidden_size >= 4096
 
 
+def _called_as_is(module: nn.Module, cls: type) -> bool:
+    """module(...) does what cls.forward does and nothing else: no subclass, no
+    replaced forward, no hook of its own or of all modules."""
+    m = nn.modules.module
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks or m._global_forward_hooks or m._global_forward_pre_hooks
+                     or m._global_backward_hooks or m._global_backward_pre_hooks))
+
+
 class LlamaAttention(nn.Module):
 
     def __init__(self, config: ModelConfig) -> None:
@@ -155,8 +165,16 @@ class LlamaAttention(nn.Module):
         qkv = self.qkv_proj(hidden_states)
         return self.o_proj(self.attend(positions, qkv))
 
+    def _one_pass_modules(self, norms: tuple) -> bool:
+        """The prefill launch that stands for the q / k norms and the rotary
+        embedding leaves their modules uncalled and (QK-norm) writes the qkv rows
+        the norms only read: not while a hook watches one of them."""
+        return (_called_as_is(self.rotary_emb, RotaryEmbedding) and all(_called_as_is(n, RMSNorm) for n in norms)
+                and not (norms and self.qkv_proj._forward_hooks))
+
     def attend(self, positions: torch.Tensor, qkv: torch.Tensor) -> torch.Tensor:
-        """Everything between the qkv and o projections; returns [T, Hq*D]."""
+        """Everything between the qkv and o projections; returns [T, Hq*D].  The
+        q and k columns of qkv may be overwritten."""
         q = qkv[:, :self.q_size].view(-1, self.num_heads, self.head_dim)
         k = qkv[:, self.q_size:self.q_size + self.kv_size].view(-1, self.num_kv_heads, self.head_dim)
         v = qkv[:, self.q_size + self.kv_size:].view(-1, self.num_kv_heads, self.head_dim)
@@ -174,6 +192,7 @@ class LlamaAttention(nn.Module):
         # prefill: QK-norm, decision and RoPE in one pass over the qkv rows (8B shape, 12 000 tokens: the
         # launches it replaces take 132 us, it takes 47)
         one_pass = (ctx.dms_capture_enabled and ctx.is_prefill and ctx.dms_layer_evictions_buffer is None
+                    and self._one_pass_modules(norms)
                     and prefill_qk_supported(q, k, self.rotary_emb.cos_sin_cache, norms))
         if self.qk_norm and not (one_launch or one_pass):  # Qwen3: QK-norm before DMS extraction (qwen3.py:92-94)
             q = self.q_norm(q)

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from native_emulator import cpu_engine
 from fastdms_amd.engine.dms import prefill_qk_supported
 from fastdms_amd.layers.layernorm import RMSNorm
 
@@ -41,3 +42,72 @@ def test_prefill_qk_refuses_rows_it_would_read_past(what):
     if what == "k width":
         k = _views(D // 2)[1]
     assert not prefill_qk_supported(q, k, table, norms)
+
+
+def _prefill(hooked=(), replace=None):
+    """Prefill logits of a two-layer QK-norm model with forward hooks on the
+    named modules of layer 1; returns (logits, hook calls, kernel calls)."""
+    with cpu_engine() as emu:
+        from fastdms_amd import LLM, SamplingParams
+        llm = LLM("tiny-qwen3", max_model_len=512, max_num_seqs=2, max_num_batched_tokens=512, enforce_eager=True,
+                  fused_greedy_head=False, dms_window_size=32, dms_alpha_scale=10.0, dms_alpha_offset=5.0)
+        attn = llm.model_runner.model.model.layers[1].self_attn
+        seen, handles = [], []
+        for name in hooked:
+            def hook(module, args, output, name=name):
+                if not (name == "qkv_proj" and seen):
+                    seen.append((name, output, output.clone() if name == "qkv_proj" else None))
+            handles.append(getattr(attn, name).register_forward_hook(hook))
+        if replace:
+            replace(attn)
+        llm.add_request(list(range(1, 150)), SamplingParams(temperature=0.0, max_tokens=2, ignore_eos=True))
+        emu.calls.clear()
+        llm.step()
+        for h in handles:
+            h.remove()
+        logits = llm.model_runner.model.lm_head.last_logits.clone()
+        calls = list(emu.calls)
+        llm.exit()
+    return logits, seen, calls
+
+
+def test_prefill_hooks_see_their_modules():
+    """A forward hook on q_norm, k_norm or rotary_emb is called at prefill, and
+    one on qkv_proj keeps rows that the norms left alone; the results stay."""
+    want, _, calls = _prefill()
+    assert calls.count("fdms_prefill_qk") == 2
+    for name in ("q_norm", "k_norm", "rotary_emb", "qkv_proj"):
+        got, seen, calls = _prefill((name,))
+        assert [s[0] for s in seen][:1] == [name]
+        # the rotary module is shared by the layers
+        assert calls.count("fdms_prefill_qk") == (0 if name == "rotary_emb" else 1)
+        assert torch.equal(got, want)
+        if name == "qkv_proj":
+            assert torch.equal(seen[0][1], seen[0][2])
+
+
+def test_prefill_runs_replaced_modules():
+    """A norm of another class, or with its own forward, is called."""
+    want, _, _ = _prefill()
+    called = []
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            called.append("class")
+            return self.inner(x)
+
+    def other_class(attn):
+        attn.q_norm = Wrapped(attn.q_norm)
+
+    def own_forward(attn):
+        plain = attn.k_norm.forward
+        attn.k_norm.forward = lambda x: (called.append("forward"), plain(x))[1]
+
+    for replace, name in ((other_class, "class"), (own_forward, "forward")):
+        got, _, _ = _prefill(replace=replace)
+        assert name in called
+        assert torch.equal(got, want)
