@@ -18,6 +18,7 @@
 // of that lane (one half swap per block, no broadcasts).  S^T's C layout is
 // the B operand of V^T . P^T once the 16 keys of a step are taken in the order
 // 8 * (i / 4) + 4 * half + i % 4, which is the order V is read in.
+#include <cfloat>
 #include <type_traits>
 
 #include "fdms_common.h"
@@ -108,16 +109,20 @@ __device__ __forceinline__ float halves_sum(float v) {
 // exponentials of block t, then V(t) . P beside the max of block t + 1.
 // Softmax rescaling is lazy: the running max only moves (and O / the sum are
 // rescaled) when a block raises it by more than 8 in the log2 domain, so p
-// stays below 256.  The running max starts at a finite floor (-1e30) instead
-// of -inf: the first block with a visible key then takes the same grow test
-// as every later one, its rescale factor exp2((floor - m) * scale) is exactly 0,
-// and a row whose keys so far are all masked keeps the floor with p = 0.
+// stays below 256.  The running max starts at a finite floor instead of -inf
+// (the lowest fp32 whose product with the scale is still finite): the first
+// block with a visible key then takes the same grow test as every later one,
+// its rescale factor exp2((floor - m) * scale) is exactly 0, and a row whose
+// keys so far all score -inf keeps the floor with p = 0.
+// The running max is of raw scores, so the softmax scale has to be positive:
+// the host hands over its magnitude, and its sign (0 for a scale of 0, with
+// the magnitude 1) multiplies Q, exactly, as the rows are read.
 template <int D, int G>
 __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
     const bf16_t* __restrict__ q, int64_t qs_t, int64_t qs_h, const bf16_t* __restrict__ k, int64_t ks_t,
     int64_t ks_h, const bf16_t* __restrict__ v, int64_t vs_t, int64_t vs_h, bf16_t* __restrict__ out, int64_t os_t,
     int64_t os_h, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, int group, int vec_out,
-    float scale_log2) {
+    float scale_log2, float q_sign, float max_floor) {
   constexpr int P = 4 * kWaveRows / G;  // query positions per workgroup
   constexpr int RB = 2 * D;             // bytes of a K / V row
   constexpr int CH = D / 8;             // 16-byte chunks of a row
@@ -187,6 +192,12 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
     const bf16_t* qp = q + (int64_t)(start + qrow) * qs_t + (int64_t)qh * qs_h + 8 * half;
 #pragma unroll
     for (int j = 0; j < KS; ++j) qop[j] = as_bf16x8(*reinterpret_cast<const uint4*>(qp + 16 * j));
+    if (q_sign != 1.0f) {  // uniform
+#pragma unroll
+      for (int j = 0; j < KS; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) qop[j][i] = (__bf16)((float)qop[j][i] * q_sign);
+    }
   }
   // LDS byte offsets of this lane's operands (buffer, key tile and key step
   // are added as constants)
@@ -203,9 +214,8 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
       vaddr[c] = vr * RB + (((4 * c + 2 * g1 + ((l16 & 3) >> 1)) ^ f) << 4) + 8 * (l16 & 1);
   }
 
-  constexpr float kMaxFloor = -1e30f;  // below any score; see the rescale note above
-  float m_run = kMaxFloor;             // raw-score running max of this lane's query
-  float l_run = 0.0f;                  // this half's share of its row sum
+  float m_run = max_floor;  // raw-score running max of this lane's query (see the rescale note above)
+  float l_run = 0.0f;       // this half's share of its row sum
   f32x16 o[DT];
 #pragma unroll
   for (int c = 0; c < DT; ++c) o[c] = f32x16{};
@@ -386,7 +396,10 @@ FDMS_EXPORT int fdms_prefill_attention_varlen(const void* q, int64_t qs_t, int64
   // token strides in elements: 64 rows of either stay in 32-bit byte offsets
   if (ks_t < 0 || vs_t < 0 || ks_t >= (1 << 24) || vs_t >= (1 << 24)) return (int)hipErrorInvalidValue;
   if (head_dim != 64 && head_dim != 128) return (int)hipErrorInvalidValue;
-  const float sl2 = scale * 1.4426950408889634f;
+  const float signed_sl2 = scale * 1.4426950408889634f;
+  const float q_sign = signed_sl2 < 0.0f ? -1.0f : signed_sl2 == 0.0f ? 0.0f : 1.0f;
+  const float sl2 = signed_sl2 == 0.0f ? 1.0f : signed_sl2 * q_sign;
+  const float max_floor = sl2 > 1.0f ? -0x1p127f / sl2 : -FLT_MAX;
   const int group = num_q_heads / num_kv_heads;
   const int packed = group == 2 || group == 4 ? group : 1;  // query heads per workgroup
   const int pos = 4 * kWaveRows / packed;                   // query positions per workgroup
@@ -395,7 +408,7 @@ FDMS_EXPORT int fdms_prefill_attention_varlen(const void* q, int64_t qs_t, int64
 #define FDMS_PREFILL(DD, GG)                                                                                       \
   hipLaunchKernelGGL((prefill_attn_kernel<DD, GG>), grid, dim3(kThreads), 0, (hipStream_t)stream, (const bf16_t*)q,  \
                      qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h, (bf16_t*)out, os_t,     \
-                     os_h, cu_seqlens_q, cu_seqlens_k, group, vec_out, sl2)
+                     os_h, cu_seqlens_q, cu_seqlens_k, group, vec_out, sl2, q_sign, max_floor)
   if (head_dim == 64) {
     if (packed == 1) FDMS_PREFILL(64, 1); else if (packed == 2) FDMS_PREFILL(64, 2); else FDMS_PREFILL(64, 4);
   } else {

@@ -292,6 +292,43 @@ def test_prefill_attention_vs_oracle(d, lens, hq, hkv, ramp):
     assert np.mean(np.abs(got - want) <= 2 ** -7 * np.abs(want) + 4e-3) > 0.99
 
 
+def _causal_attention64(q, k, v, lens, scale):
+    """Causal attention of a ragged batch in 64 bits; q [T, Hq, D], k / v [T, Hkv, D]."""
+    out, a = [], 0
+    group = q.shape[1] // k.shape[1]
+    for n in lens:
+        qs, ks, vs = (x[a:a + n].double().transpose(0, 1) for x in (q, k, v))
+        ks, vs = ks.repeat_interleave(group, 0), vs.repeat_interleave(group, 0)
+        s = (qs @ ks.transpose(1, 2)) * scale
+        s = s.masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), -float("inf"))
+        out.append((torch.softmax(s, -1) @ vs).transpose(0, 1))
+        a += n
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("hq,hkv", [(4, 4), (8, 4), (8, 2), (6, 2), (16, 2)])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 1.5, "low"])
+def test_prefill_attention_scales(d, hq, hkv, scale):
+    """Softmax scales of either sign, 0 and above 1, and raw scores that all lie
+    near -1e32 (the running max starts below them), at every way a group of
+    query heads is run.  Tolerance: P and the output rounded to bf16 (2^-9
+    each) against values of RMS below 1."""
+    require_gpu()
+    from fastdms_amd.layers.attention import prefill_attention
+    lens = [1, 64, 65, 200]
+    g = torch.Generator().manual_seed(d + hq * hkv)
+    q, k, v = (torch.randn(sum(lens), h, d, generator=g) for h in (hq, hkv, hkv))
+    if scale == "low":
+        q, k, scale = q * 1e14 + 1e15, k * 1e14 - 1e16, 0.5e-30
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    want = _causal_attention64(q, k, v, lens, scale)
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    got = prefill_attention(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), max(lens), scale).double().cpu()
+    assert torch.isfinite(got).all()
+    assert float((got - want).abs().max()) <= 2 ** -7 * max(1.0, float(want.abs().max()))
+
+
 @pytest.mark.parametrize("hq,hkv", [(8, 2), (8, 4), (4, 4)])
 def test_prefill_attention_query_tiles_agree(hq, hkv, monkeypatch):
     """The packed kernel with two or four 16-row query tiles per wave (four
