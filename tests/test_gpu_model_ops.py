@@ -329,6 +329,36 @@ def test_prefill_attention_scales(d, hq, hkv, scale):
     assert float((got - want).abs().max()) <= 2 ** -7 * max(1.0, float(want.abs().max()))
 
 
+@pytest.mark.parametrize("d,hq,hkv,sum32", [(64, 6, 2, True), (128, 16, 2, True), (128, 5, 1, True),
+                                            (64, 8, 2, False), (128, 4, 4, False)])
+def test_prefill_attention_row_sum_width(d, hq, hkv, sum32):
+    """The softmax denominator: fp32 probabilities for group sizes other than 1,
+    2 and 4, the numerator's bf16 ones for those.  Rows of at most 12 keys, where
+    the two differ most; of the outputs that round differently under the two
+    (each computed in 64 bits around the bf16 probabilities), at least nine in
+    ten are those of the kind that runs (fp32 scores put a few on the other side
+    of a rounding boundary)."""
+    require_gpu()
+    from fastdms_amd.layers.attention import prefill_attention
+    lens, scale = [12] * 400, d ** -0.5
+    g = torch.Generator().manual_seed(d * hq)
+    q, k, v = (torch.randn(sum(lens), h, d, generator=g).to(torch.bfloat16) for h in (hq, hkv, hkv))
+    n, group = 12, hq // hkv
+    qs, ks, vs = (x.double().view(-1, n, x.shape[1], d).transpose(1, 2) for x in (q, k, v))
+    ks, vs = ks.repeat_interleave(group, 1), vs.repeat_interleave(group, 1)
+    s = (qs @ ks.transpose(2, 3)).masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), -float("inf"))
+    p = torch.exp((s - s.amax(-1, keepdim=True)) * scale)
+    p16 = p.float().to(torch.bfloat16).double()
+    num = p16 @ vs
+    of = {True: num / p.sum(-1, keepdim=True), False: num / p16.sum(-1, keepdim=True)}
+    of = {w: o.transpose(1, 2).reshape(-1, hq, d).float().to(torch.bfloat16) for w, o in of.items()}
+    cu = torch.arange(len(lens) + 1, dtype=torch.int32) * n
+    got = prefill_attention(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), n, scale).cpu()
+    split = of[True] != of[False]
+    assert int(split.sum()) > 10000
+    assert float((got == of[sum32])[split].float().mean()) > 0.9
+
+
 @pytest.mark.parametrize("hq,hkv", [(8, 2), (8, 4), (4, 4)])
 def test_prefill_attention_query_tiles_agree(hq, hkv, monkeypatch):
     """The packed kernel with two or four 16-row query tiles per wave (four
