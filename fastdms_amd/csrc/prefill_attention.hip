@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "fdms_common.h"
+#include "fdms_prefill_blocks.h"
 
 using namespace fdms;
 
@@ -33,9 +34,9 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kKeys = 64;    // keys per LDS block
+constexpr int kKeys = kPrefillKeys;  // keys per LDS block
 constexpr int kThreads = 256;
-constexpr int kWaveRows = 32;  // query rows per wave
+constexpr int kWaveRows = kPrefillWaveRows;  // query rows per wave
 
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
   bf16x8 r;
@@ -162,11 +163,11 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
   const int lc = lane & 31, half = lane >> 5;
   const int qh = hg * G + wave % G;
   const int kvh = (hg * G) / group;
-  const int wq0 = q0 + (wave / G) * kWaveRows;                  // first position of this wave
-  const int wq_last = min(wq0 + kWaveRows - 1, len - 1);        // last valid position of this wave
-  const int kend = min(klen, off + q0 + P);                     // keys some row of the workgroup sees
-  const int nkb = (kend + kKeys - 1) / kKeys;
-  const int nw = wq0 < len ? (off + wq_last) / kKeys + 1 : 0;   // blocks this wave sees (<= nkb)
+  const int wq0 = q0 + (wave / G) * kWaveRows;  // first position of this wave
+  // blocks the workgroup loads, this wave sees, and every row of it sees whole
+  // (the others need the mask); a wave past the sequence only loads its share
+  const PrefillBlocks blocks = prefill_blocks(len, klen, q0, P, wq0);
+  const int nkb = blocks.loaded, nw = blocks.seen, nfull = blocks.whole;
 
   const uint8_t* kbase = reinterpret_cast<const uint8_t*>(k + (int64_t)kstart * ks_t + (int64_t)kvh * ks_h);
   const uint8_t* vbase = reinterpret_cast<const uint8_t*>(v + (int64_t)kstart * vs_t + (int64_t)kvh * vs_h);
@@ -308,8 +309,6 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
       }
   };
 
-  // blocks every row of the wave sees whole: the others need the mask
-  const int nfull = min((off + wq0 + 1) / kKeys, klen / kKeys);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), known to the compiler: Q has landed, no use of it waits again
   lds_dma_barrier();
   if (nw > 0) {

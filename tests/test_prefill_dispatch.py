@@ -1,4 +1,9 @@
-"""Which prefill layers take q and k through the one-pass launch (fdms_prefill_qk)."""
+"""Which prefill layers take q and k through the one-pass launch
+(fdms_prefill_qk), and which key blocks a prefill attention wave works on."""
+import shutil
+import subprocess
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -111,3 +116,17 @@ def test_prefill_runs_replaced_modules():
         got, _, _ = _prefill(replace=replace)
         assert name in called
         assert torch.equal(got, want)
+
+
+def test_prefill_attention_block_ranges(tmp_path):
+    """Every row's visible keys and no others, the same barriers in every wave of
+    a workgroup, no work in a wave past the sequence's end."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    root = Path(__file__).resolve().parents[1]
+    exe = tmp_path / "prefill_blocks_check"
+    subprocess.run([gxx, "-std=c++17", "-O1", "-I", str(root / "fastdms_amd" / "csrc"),
+                    str(root / "tests" / "prefill_blocks_check.cpp"), "-o", str(exe)], check=True)
+    res = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert res.returncode == 0 and res.stdout.strip() == "ok", res.stdout + res.stderr
