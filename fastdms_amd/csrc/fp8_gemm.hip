@@ -23,6 +23,7 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 
 constexpr int kGemmXcds = 8;
 
@@ -236,13 +237,19 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void fp8_gemm_tile_kernel(
         for (int q = 0; q < 2; ++q) {
           const auto s0 = __builtin_amdgcn_permlane32_swap(o[4 * q], o[4 * q + 2], false, false);
           const auto s1 = __builtin_amdgcn_permlane32_swap(o[4 * q + 1], o[4 * q + 3], false, false);
-          if (m < M) *reinterpret_cast<uint4*>(yr + nt + 16 * q + 8 * half) = uint4{s0[0], s1[0], s0[1], s1[1]};
+          if (m < M) *reinterpret_cast<u32x4_a8*>(yr + nt + 16 * q + 8 * half) = u32x4_a8{s0[0], s1[0], s0[1], s1[1]};
         }
       } else if (m < M) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int n = nt + 8 * (r / 4) + 4 * half + r % 4;
-          if (n < N) yr[n].bits = (uint16_t)(o[r / 2] >> (16 * (r & 1)));
+        for (int r = 0; r < 16; r += 4) {
+          const int n = nt + 8 * (r / 4) + 4 * half;
+          if (VEC_OUT && n + 3 < N) {
+            *reinterpret_cast<uint2*>(yr + n) = uint2{o[r / 2], o[r / 2 + 1]};
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < N) yr[n + e].bits = (uint16_t)(o[(r + e) / 2] >> (16 * (e & 1)));
+          }
         }
       }
     }
@@ -262,7 +269,9 @@ FDMS_EXPORT int fdms_fp8_gemm(const void* x, int64_t x_s, const float* x_inv, co
   if (M == 0) return 0;
   if (!x || !x_inv || !w || !w_inv || !y) return (int)hipErrorInvalidValue;
   if (((uintptr_t)x | (uintptr_t)w) & 15) return (int)hipErrorInvalidValue;
-  const bool vec = (y_s % 8) == 0 && ((uintptr_t)y % 16) == 0;
+  // 8-byte aligned rows: whole 32-column tiles leave as 16-byte stores (a global store needs 4-byte alignment),
+  // the last columns as 8-byte ones (12000 x 16384 x 2048 with a row stride of 16388: 494 us, 810 in 2-byte stores)
+  const bool vec = (y_s % 4) == 0 && ((uintptr_t)y % 8) == 0;
 #define FDMS_GEMM_TILE(B, V, ...)                                                                                  \
   hipLaunchKernelGGL((fp8_gemm_tile_kernel<B, V, __VA_ARGS__>), grid, dim3(threads), 0, (hipStream_t)stream,        \
                      (const uint8_t*)x, x_s, x_inv, (const uint8_t*)w, w_s, w_inv, (const bf16_t*)bias, (bf16_t*)y,  \
