@@ -77,6 +77,11 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   const bf16x2_t r = {(__bf16)a, (__bf16)b};
   return __builtin_bit_cast(uint32_t, r);
 }
+// bytes 0 and 1 (HI: 2 and 3) of w, each an INT4 code 0 .. 15, as fp32 (see the INT4 branch of the kernel)
+template <bool HI>
+__device__ __forceinline__ auto codes2(int w) {
+  return __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w, 512.0f, HI);
+}
 __device__ __forceinline__ float rbf(float a) { return (float)(__bf16)a; }  // round to bf16
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
@@ -441,22 +446,23 @@ __global__ __launch_bounds__(NW * 64) void linear_small_m_kernel(
           // w = bf16((q - 8) * s + z) as one fma of the code: q * s + (z - 8s)
           // (z - 8s exact for the symmetric zero 0).  A byte 0x0q read as e4m3fn
           // is q * 2^-9 for every code (subnormal below 8), so one
-          // v_cvt_pk_f32_fp8 converts two codes, exactly (19 vector instructions
-          // per eight weights; with one v_cvt_f32_ubyte per code 22, and the
-          // group index by a division: gate_up of the 8B shape at four rows
-          // 21.0 -> 20.0 us, bound by the issue and latency of its loads)
+          // v_cvt_scalef32_pk_f32_fp8 with the scale 2^9 converts two codes,
+          // exactly (19 vector instructions per eight weights; with one
+          // v_cvt_f32_ubyte per code 22, and the group index by a division:
+          // gate_up of the 8B shape at four rows 21.0 -> 20.0 us, bound by the
+          // issue and latency of its loads).  The 2^9 is not folded into s,
+          // which would overflow from 2^119 on.
           const float sc = bf_lo(b.gsz[a][u]), zc = bf_hi(b.gsz[a][u]);
-          const float c8 = __builtin_fmaf(-8.0f, sc, zc), s9 = sc * 512.0f;
+          const float c8 = __builtin_fmaf(-8.0f, sc, zc);
           const uint32_t wd[4] = {b.w4[a][u].x, b.w4[a][u].y, b.w4[a][u].z, b.w4[a][u].w};
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int lo = (int)(wd[j] & 0x0F0F0F0Fu), hi = (int)((wd[j] >> 4) & 0x0F0F0F0Fu);
-            const auto l0 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), l1 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, true);
-            const auto h0 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, false), h1 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, true);
-            const uint4 aw = uint4{pack2(__builtin_fmaf(l0[0], s9, c8), __builtin_fmaf(h0[0], s9, c8)),
-                                   pack2(__builtin_fmaf(l0[1], s9, c8), __builtin_fmaf(h0[1], s9, c8)),
-                                   pack2(__builtin_fmaf(l1[0], s9, c8), __builtin_fmaf(h1[0], s9, c8)),
-                                   pack2(__builtin_fmaf(l1[1], s9, c8), __builtin_fmaf(h1[1], s9, c8))};
+            const auto l0 = codes2<false>(lo), l1 = codes2<true>(lo), h0 = codes2<false>(hi), h1 = codes2<true>(hi);
+            const uint4 aw = uint4{pack2(__builtin_fmaf(l0[0], sc, c8), __builtin_fmaf(h0[0], sc, c8)),
+                                   pack2(__builtin_fmaf(l0[1], sc, c8), __builtin_fmaf(h0[1], sc, c8)),
+                                   pack2(__builtin_fmaf(l1[0], sc, c8), __builtin_fmaf(h1[0], sc, c8)),
+                                   pack2(__builtin_fmaf(l1[1], sc, c8), __builtin_fmaf(h1[1], sc, c8))};
             acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(aw), as_bf16x8(bxs[j]), acc[a], 0, 0, 0);
           }
         }

@@ -577,6 +577,30 @@ def test_linear_int4_small_m_matches_oracle(m, n, k, group, mode):
                     ulps=2.0, atol=2e-3)
 
 
+def test_linear_int4_scales_over_their_whole_range():
+    """Group scales from 2^-133 (subnormal) to 2^122, one power of two per weight
+    row, every code: (q - 8) * s is exact in bf16 (or, subnormal, rounded once),
+    so the products are too, and the fp32 sums of 512 of them stay finite.
+    Tolerance: fp32 sums (2^-24 of the sum of magnitudes per addition at most)
+    and the bf16 output (8 significant bits: 2^-8 of the value, and half the
+    smallest subnormal)."""
+    require_gpu()
+    from fastdms_amd.layers.linear import linear_int4_small_m
+    exps = torch.arange(-133, 123)
+    n, k, m = len(exps), 512, 3
+    g = torch.Generator().manual_seed(2)
+    q = torch.randint(0, 16, (n, k), generator=g)
+    x = torch.randint(-8, 9, (m, k), generator=g).to(torch.bfloat16) * 2.0 ** -8
+    sz = torch.zeros(k // 128, n, 2, dtype=torch.bfloat16)
+    sz[..., 0] = torch.ldexp(torch.ones(n, dtype=torch.float64), exps).to(torch.bfloat16)
+    packed = (q[:, 0::2] | (q[:, 1::2] << 4)).to(torch.uint8)
+    w = ((q - 8).double() * sz[0, :, 0].double()[:, None]).to(torch.bfloat16).double()
+    want, mag = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+    y = linear_int4_small_m(x.cuda(), packed.cuda(), sz.cuda(), 128).double().cpu()
+    assert torch.isfinite(y).all()
+    assert bool(((y - want).abs() <= 2.0 ** -8 * want.abs() + 512 * 2.0 ** -24 * mag + 2.0 ** -134).all())
+
+
 @pytest.mark.parametrize("splits", [1, 2, 4])
 def test_int4_partials_equal_the_merged_linear(splits):
     """W4A16 epilogue 3: the fp32 split partials summed in split order are the

@@ -312,8 +312,8 @@ def _causal_attention64(q, k, v, lens, scale):
 def test_prefill_attention_scales(d, hq, hkv, scale):
     """Softmax scales of either sign, 0 and above 1, and raw scores that all lie
     near -1e32 (the running max starts below them), at every way a group of
-    query heads is run.  Tolerance: P and the output rounded to bf16 (2^-9
-    each) against values of RMS below 1."""
+    query heads is run.  Tolerance: P and the output rounded to bf16 (8
+    significant bits, 2^-8 each) of values of at most the largest output."""
     require_gpu()
     from fastdms_amd.layers.attention import prefill_attention
     lens = [1, 64, 65, 200]
