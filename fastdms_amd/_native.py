@@ -46,6 +46,7 @@ SIGNATURES: dict[str, str] = {
     "fdms_record_dms_decisions": "pllllpllllplllplllpipiiiip",
     "fdms_argmax_rows": "pillipp",
     "fdms_mfma_probe": "pppp",
+    "fdms_prefill_mfma_probe": "ippppppp",
     "fdms_prefill_attention": "pllpllpllpllpiiiiifp",
     "fdms_prefill_attention_varlen": "pllpllpllpllppiiiiifp",
     "fdms_rmsnorm": "pllippplplifpplip",

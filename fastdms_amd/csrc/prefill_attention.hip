@@ -80,14 +80,45 @@ __device__ __forceinline__ float halves_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// K/V rows in LDS are row-major and unpadded with the 16-byte chunks of a row
+// XOR-swizzled.  K: chunk c of row r at slot c ^ (r & 15) (head_dim 128; (r / 2)
+// & 7 at 64), so the 32 rows of an A operand spread over all banks.  V: chunk c
+// at slot c ^ 4 * (r & 3) (4 * ((r / 2) & 1)); its A operand is read with the
+// transposing ds_read_b64_tr_b16 (16 lanes: four keys x 16 dims).
+template <int D>
+__device__ __forceinline__ int k_swizzle(int row) {
+  return D == 128 ? row & 15 : (row >> 1) & 7;
+}
+template <int D>
+__device__ __forceinline__ int v_swizzle(int row) {
+  return D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2;
+}
+// Byte offset of a lane's part of the K operand (32 keys x 16 dims from dim 16 j).
+template <int D>
+__device__ __forceinline__ uint32_t k_operand(int lane, int j) {
+  const int row = lane & 31;
+  return row * 2 * D + (((2 * j + (lane >> 5)) ^ k_swizzle<D>(row)) << 4);
+}
+// Byte offset of a lane's first read of the V operand (32 dims from dim 32 c x the
+// first 16 keys): l16 its place in its group of 16, g1 the group's half of the
+// dims, row = v_row(l16, lane / 32); the second read is eight rows on.
+__device__ __forceinline__ int v_row(int l16, int half) { return 4 * half + (l16 >> 2); }
+template <int D>
+__device__ __forceinline__ uint32_t v_operand(int row, int l16, int g1, int c) {
+  return row * 2 * D + (((4 * c + 2 * g1 + ((l16 & 3) >> 1)) ^ v_swizzle<D>(row)) << 4) + 8 * (l16 & 1);
+}
+// The two transposing reads of a V operand at LDS byte address `at`, rows of `row_bytes`.
+__device__ __forceinline__ bf16x8 read_v(uint32_t at, int row_bytes) {
+  using lds_s16x4 = __attribute__((address_space(3))) s16x4;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)at);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(at + 8 * row_bytes));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 }  // namespace
 
-// K/V blocks go from global memory straight into LDS, row-major and unpadded
-// with the 16-byte chunks of a row XOR-swizzled (the lane picks which chunk it
-// loads), double-buffered.  K: chunk c of row r at slot c ^ (r & 15) (head_dim
-// 128; (r / 2) & 7 at 64), so the 32 rows of an A operand spread over all
-// banks.  V: chunk c at slot c ^ 4 * (r & 3) (4 * ((r / 2) & 1)); its A operand is
-// read with the transposing ds_read_b64_tr_b16 (16 lanes: four keys x 16 dims).
+// K/V blocks go from global memory straight into LDS (the lane picks which
+// chunk it loads, see the swizzles above), double-buffered.
 //
 // What bounds it: power and the matrix cores together -- the clock falls to
 // 1.8 GHz while it runs (2.35 GHz under a memory-bound kernel) with the matrix
@@ -175,8 +206,8 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
   // this lane's part of an LDS-DMA instruction: row drow (+ 4 * RPI * i), the
   // chunk whose swizzled slot is lane % CH
   const int drow = wave * RPI + lane / CH;
-  const int kchunk = (lane % CH) ^ (D == 128 ? drow & 15 : (drow >> 1) & 7);
-  const int vchunk = (lane % CH) ^ (D == 128 ? (drow & 3) << 2 : ((drow >> 1) & 1) << 2);
+  const int kchunk = (lane % CH) ^ k_swizzle<D>(drow);
+  const int vchunk = (lane % CH) ^ v_swizzle<D>(drow);
   const uint32_t ksb = (uint32_t)(ks_t * 2), vsb = (uint32_t)(vs_t * 2);  // row strides in bytes
   auto load_tile = [&](const uint8_t* base, uint32_t stride, int chunk, int blk, uint32_t lds) {
     const int k0 = blk * kKeys;
@@ -210,15 +241,12 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
   // are added as constants)
   uint32_t kaddr[KS], vaddr[DT];
 #pragma unroll
-  for (int j = 0; j < KS; ++j)
-    kaddr[j] = lc * RB + (((2 * j + half) ^ (D == 128 ? lc & 15 : (lc >> 1) & 7)) << 4);
+  for (int j = 0; j < KS; ++j) kaddr[j] = k_operand<D>(lane, j);
   {
     const int l16 = lane & 15, g1 = (lane >> 4) & 1;
-    const int vr = 4 * half + (l16 >> 2);
-    const int f = D == 128 ? (vr & 3) << 2 : ((vr >> 1) & 1) << 2;
+    const int vr = v_row(l16, half);
 #pragma unroll
-    for (int c = 0; c < DT; ++c)
-      vaddr[c] = vr * RB + (((4 * c + 2 * g1 + ((l16 & 3) >> 1)) ^ f) << 4) + 8 * (l16 & 1);
+    for (int c = 0; c < DT; ++c) vaddr[c] = v_operand<D>(vr, l16, g1, c);
   }
 
   float m_run = max_floor;  // raw-score running max of this lane's query (see the rescale note above)
@@ -295,18 +323,12 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(
     }
   };
   auto pv = [&](const uint4 (&pb)[4], int buf) {
-    using lds_s16x4 = __attribute__((address_space(3))) s16x4;
     const uint32_t vt = lds0 + (2 + buf) * TILE;
 #pragma unroll
     for (int st = 0; st < 4; ++st)
 #pragma unroll
-      for (int c = 0; c < DT; ++c) {
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(vt + vaddr[c] + (16 * st) * RB));
-        const s16x4 hi =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(vt + vaddr[c] + (16 * st + 8) * RB));
-        const auto both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        o[c] = mfma32x32x16(__builtin_bit_cast(bf16x8, both), as_bf16x8(pb[st]), o[c]);
-      }
+      for (int c = 0; c < DT; ++c)
+        o[c] = mfma32x32x16(read_v(vt + vaddr[c] + (16 * st) * RB, RB), as_bf16x8(pb[st]), o[c]);
   };
 
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), known to the compiler: Q has landed, no use of it waits again
@@ -439,7 +461,7 @@ FDMS_EXPORT int fdms_prefill_attention(const void* q, int64_t qs_t, int64_t qs_h
 }
 
 // One v_mfma_f32_16x16x32_bf16 of a 16x32 A and a 32x16 B (row-major bf16)
-// loaded with the operand layout the kernels above assume; C row-major fp32.
+// loaded with the operand layout the decode linears assume; C row-major fp32.
 // Exists so a test can confirm that layout against a host matmul.
 __global__ void mfma_probe_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b, float* __restrict__ c) {
   const int l = threadIdx.x;
@@ -461,6 +483,60 @@ FDMS_EXPORT int fdms_mfma_probe(const void* a, const void* b, float* c, void* st
   if (!a || !b || !c) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(mfma_probe_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, (const bf16_t*)a,
                      (const bf16_t*)b, c);
+  FDMS_LAUNCH_CHECK();
+  return 0;
+}
+
+// The prefill kernel's two products through its own operand addresses: S^T [32
+// keys, 32 queries] = K . Q^T of k, q [32, D], and O [32 queries, D] = P . V of p
+// [32 queries, 16 keys], v [16 keys, D], V read transposed in the permuted key
+// order.  One wave; exists so a test can confirm the layouts against host matmuls.
+template <int D>
+__global__ void prefill_mfma_probe_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ q,
+                                          float* __restrict__ s, const bf16_t* __restrict__ p,
+                                          const bf16_t* __restrict__ v, float* __restrict__ o) {
+  constexpr int RB = 2 * D, CH = D / 8;
+  __shared__ __attribute__((aligned(1024))) uint8_t s_k[32 * RB], s_v[16 * RB];
+  const int lane = threadIdx.x, lc = lane & 31, half = lane >> 5;
+  for (int u = lane; u < 32 * CH; u += kWave)
+    *reinterpret_cast<uint4*>(s_k + (u / CH) * RB + (((u % CH) ^ k_swizzle<D>(u / CH)) << 4)) =
+        reinterpret_cast<const uint4*>(k)[u];
+  for (int u = lane; u < 16 * CH; u += kWave)
+    *reinterpret_cast<uint4*>(s_v + (u / CH) * RB + (((u % CH) ^ v_swizzle<D>(u / CH)) << 4)) =
+        reinterpret_cast<const uint4*>(v)[u];
+  __syncthreads();
+  f32x16 acc{};
+  for (int j = 0; j < D / 16; ++j)
+    acc = mfma32x32x16(as_bf16x8(*reinterpret_cast<const uint4*>(s_k + k_operand<D>(lane, j))),
+                       as_bf16x8(*reinterpret_cast<const uint4*>(q + lc * D + 16 * j + 8 * half)), acc);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s[(8 * (r / 4) + 4 * half + r % 4) * 32 + lc] = acc[r];
+  uint16_t pv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) pv[i] = p[lc * 16 + 8 * (i / 4) + 4 * half + i % 4].bits;
+  uint4 pb;
+  __builtin_memcpy(&pb, pv, 16);
+  const uint32_t vt = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)s_v;
+  const int l16 = lane & 15, g1 = (lane >> 4) & 1;
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    const uint32_t at = vt + v_operand<D>(v_row(l16, half), l16, g1, c);
+    acc = mfma32x32x16(read_v(at, RB), as_bf16x8(pb), f32x16{});
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[lc * D + 32 * c + 8 * (r / 4) + 4 * half + r % 4] = acc[r];
+  }
+}
+
+FDMS_EXPORT int fdms_prefill_mfma_probe(int head_dim, const void* k, const void* q, float* s, const void* p,
+                                        const void* v, float* o, void* stream) {
+  if (!k || !q || !s || !p || !v || !o || (head_dim != 64 && head_dim != 128) || !fdms_aligned16(k, q, v))
+    return (int)hipErrorInvalidValue;
+  if (head_dim == 64)
+    hipLaunchKernelGGL(prefill_mfma_probe_kernel<64>, dim3(1), dim3(kWave), 0, (hipStream_t)stream, (const bf16_t*)k,
+                       (const bf16_t*)q, s, (const bf16_t*)p, (const bf16_t*)v, o);
+  else
+    hipLaunchKernelGGL(prefill_mfma_probe_kernel<128>, dim3(1), dim3(kWave), 0, (hipStream_t)stream, (const bf16_t*)k,
+                       (const bf16_t*)q, s, (const bf16_t*)p, (const bf16_t*)v, o);
   FDMS_LAUNCH_CHECK();
   return 0;
 }

@@ -286,9 +286,16 @@ int fdms_prefill_attention_varlen(const void* q, int64_t qs_t, int64_t qs_h, con
                                   int num_seqs, int max_seqlen_q, int num_q_heads, int num_kv_heads, int head_dim,
                                   float scale, void* stream);
 
-/* One v_mfma_f32_16x16x32_bf16 with the operand layout the attention kernels
+/* One v_mfma_f32_16x16x32_bf16 with the operand layout the decode linears
  * assume (no reference counterpart: a lane-layout self-check for tests). */
 int fdms_mfma_probe(const void* a, const void* b, float* c, void* stream);
+
+/* The prefill attention's two products on one wave, through its own operand
+ * layouts and LDS swizzles (no reference counterpart: a self-check for tests).
+ * head_dim D 64 or 128; k, q [32, D], p [32, 16], v [16, D] bf16 (k, q, v 16-byte
+ * aligned) -> s [32, 32] = k q^T, o [32, D] = p v, fp32. */
+int fdms_prefill_mfma_probe(int head_dim, const void* k, const void* q, float* s, const void* p, const void* v,
+                            float* o, void* stream);
 
 /* Residual-add + RMSNorm, bf16 (fastdms/layers/layernorm.py:16-40).  Row r of the
  * input is at in + (r/heads)*in_stride + (r%heads)*in_head_stride (heads > 1

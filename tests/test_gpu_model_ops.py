@@ -17,7 +17,7 @@ def _bf16(x: np.ndarray) -> torch.Tensor:
 
 
 def test_mfma_operand_layout():
-    """v_mfma_f32_16x16x32_bf16 with the lane layout the prefill kernel assumes.
+    """v_mfma_f32_16x16x32_bf16 with the lane layout the decode linears assume.
     Small integers keep every product and sum exact, so the check is exact."""
     require_gpu()
     from fastdms_amd import _native as nat
@@ -29,6 +29,25 @@ def test_mfma_operand_layout():
     nat.call("fdms_mfma_probe", ad.data_ptr(), bd.data_ptr(), c.data_ptr(), nat.stream())
     torch.cuda.synchronize()
     np.testing.assert_array_equal(c.cpu().numpy(), a @ b)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_operand_layouts(d):
+    """The prefill kernel's v_mfma_f32_32x32x16_bf16 operands: K rows from
+    swizzled LDS against Q rows, V rows through the transposing LDS read against P
+    in the permuted key order.  Small integers keep every sum exact."""
+    require_gpu()
+    from fastdms_amd import _native as nat
+    rng = np.random.default_rng(d)
+    k, q, p, v = (rng.integers(-3, 4, shape).astype(np.float32) for shape in ((32, d), (32, d), (32, 16), (16, d)))
+    kd, qd, pd, vd = (_bf16(x).cuda() for x in (k, q, p, v))
+    s = torch.empty((32, 32), device="cuda", dtype=torch.float32)
+    o = torch.empty((32, d), device="cuda", dtype=torch.float32)
+    nat.call("fdms_prefill_mfma_probe", d, kd.data_ptr(), qd.data_ptr(), s.data_ptr(), pd.data_ptr(), vd.data_ptr(),
+             o.data_ptr(), nat.stream())
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(s.cpu().numpy(), k @ q.T)
+    np.testing.assert_array_equal(o.cpu().numpy(), p @ v)
 
 
 def _rms_ref(x, w, eps, residual=None):
@@ -253,9 +272,9 @@ def test_argmax_rows_matches_torch(dtype):
 @pytest.mark.parametrize("d,lens,hq,hkv,ramp", [
     (64, [1, 63, 64, 65, 200, 517], 8, 2, 0.0),
     (128, [129, 700, 2], 8, 2, 0.0),
-    (64, [31, 160, 1500], 4, 4, 0.0),      # G = 1 (packed kernel, 128 positions per workgroup)
+    (64, [31, 160, 1500], 4, 4, 0.0),      # G = 1 (128 positions per workgroup)
     (128, [95, 300], 8, 4, 0.0),           # G = 2
-    (64, [77, 400], 6, 2, 0.0),            # G = 3 (per-head kernel)
+    (64, [77, 400], 6, 2, 0.0),            # G = 3 (one query head per workgroup)
     (64, [2100, 130], 8, 2, 3.0),          # keys scaled up along the sequence: the running max keeps growing
     (128, [900], 8, 2, 3.0),
 ])
@@ -359,13 +378,11 @@ def test_prefill_attention_row_sum_width(d, hq, hkv, sum32):
     assert float((got == of[sum32])[split].float().mean()) > 0.9
 
 
-@pytest.mark.parametrize("hq,hkv", [(8, 2), (8, 4), (4, 4)])
-def test_prefill_attention_query_tiles_agree(hq, hkv, monkeypatch):
-    """The packed kernel with two or four 16-row query tiles per wave (four
-    is selectable at head_dim 64): each row's arithmetic is the same, only a
-    workgroup's span of positions differs, so the outputs are bit-identical,
-    and both match the oracle.  Keys grow along the sequence, so the lazy
-    rescale runs after the first block."""
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (8, 4), (4, 4), (6, 2), (8, 1)])
+def test_prefill_attention_rescales_as_keys_grow(hq, hkv):
+    """Keys grow along the sequence, so later blocks raise a row's running max by
+    more than the lazy rescale lets pass, again and again: every way a group of
+    query heads is run matches the oracle."""
     require_gpu()
     from fastdms_amd.layers.attention import prefill_attention
     d, lens = 64, [1, 700, 1500, 64, 129]
@@ -384,13 +401,9 @@ def test_prefill_attention_query_tiles_agree(hq, hkv, monkeypatch):
     qd = dq[:, :hq * d].view(t, hq, d)
     kd = dq[:, hq * d:(hq + hkv) * d].view(t, hkv, d)
     vd = dq[:, (hq + hkv) * d:].view(t, hkv, d)
-    outs = {}
-    for qt in ("2", "4"):
-        monkeypatch.setenv("FASTDMS_AMD_PREFILL_QT", qt)
-        outs[qt] = prefill_attention(qd, kd, vd, torch.from_numpy(cu).cuda(), max(lens), d ** -0.5)
-        torch.cuda.synchronize()
-    assert torch.equal(outs["2"], outs["4"])
-    got = outs["4"].float().cpu().numpy()
+    out = prefill_attention(qd, kd, vd, torch.from_numpy(cu).cuda(), max(lens), d ** -0.5)
+    torch.cuda.synchronize()
+    got = out.float().cpu().numpy()
     err = np.abs(got - want).max() / np.abs(want).max()
     assert err <= 2e-2, f"max-abs-rel error {err:.3g}"
     assert np.mean(np.abs(got - want) <= 2 ** -7 * np.abs(want) + 4e-3) > 0.99
@@ -437,7 +450,7 @@ def test_prefill_attention_block_edges(d, hq, hkv, blocks, pad):
     (128, [700, 129], [511, 128], 8, 2),
     (64, [1500, 90], [1499, 37], 4, 4),           # G = 1, a one-row chunk
     (128, [400], [3], 8, 4),                      # G = 2
-    (64, [333, 200], [200, 1], 6, 2),             # G = 3 (per-head kernel)
+    (64, [333, 200], [200, 1], 6, 2),             # G = 3 (one query head per workgroup)
 ])
 def test_prefill_attention_chunk_over_retained_prefix(d, lens, cuts, hq, hkv):
     """A prompt chunk attending to the retained earlier chunks plus itself
