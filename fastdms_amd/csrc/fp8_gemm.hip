@@ -118,7 +118,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void fp8_gemm_tile_kernel(
   for (int i = 0; i < NWI; ++i) woff[i] = (Off)min(16 * (i * NW + wave) + drow, N - 1 - nb0) * (Off)w_s;
   const uint8_t* xb = x + (int64_t)mb * x_s;
   const uint8_t* wb = w + (int64_t)nb0 * w_s;
-  const int nst = (K + kStage - 1) / kStage;
+  const int nst = K / kStage + (K % kStage != 0);  // K may be near 2^31
   auto load_stage = [&](int st) {
     const uint32_t buf = lds0 + (uint32_t)(st % NS) * (XB + WB);
     const int k0 = st * kStage;
