@@ -52,14 +52,16 @@ __device__ __forceinline__ i32x8 as_i32x8(const uint4& a, const uint4& b) {
 // at slot q ^ ((r / 4) & 3)), so the 16 rows a fragment read touches at a time
 // spread over the banks.
 //
-// What bounds it: the latency of a stage's loads while few workgroups run, the
-// matrix cores and the LDS reads (96 of 128 bytes a cycle at the 256 x 256
-// tile) once the chip is full; at K = 2048 a tile's prologue and epilogue are
-// about a sixth of its time.  Measured with the row quantisation in front
-// (M x N x K, against register-staged 256 x 256 tiles of four waves with one
-// k-block in flight): 12000 x 16384 x 2048 1 033 -> 444 us (1.86 PFLOP/s), 8192 x
-// 24576 x 4096 1 615 -> 816 us, 12000 x 2048 x 2048 180 -> 79 us, 1500 x 4096 x 4096
-// 140 -> 43 us, 64 x 2048 x 8192 104 -> 29 us.
+// What bounds it: the latency of a stage's loads while few workgroups run.  Once
+// the chip is full the matrix cores are 43 % busy (counters at 12000 x 16384 x
+// 2048, clock 2.0 GHz, no LDS bank conflicts; the fragment reads would take 96 of
+// 128 bytes a cycle at full matrix rate), so neither they nor LDS is saturated:
+// what is left is the barrier per 64-byte stage and, at K = 2048, a tile's
+// prologue and epilogue.  Measured with the row quantisation in front (M x N x K,
+// against register-staged 256 x 256 tiles of four waves with one k-block in
+// flight): 12000 x 16384 x 2048 1 019 -> 455 us (1.77 PFLOP/s; the GEMM alone 418
+// us, 1.93), 8192 x 24576 x 4096 1 563 -> 831 (1.98), 12000 x 2048 x 2048 181 -> 80,
+// 1500 x 4096 x 4096 141 -> 45, 64 x 2048 x 8192 105 -> 30.
 namespace {
 constexpr int kStage = 64;  // bytes of a row per stage
 constexpr int kGroupM = 4;  // x tiles that share a run of w tiles (4 x 8 tiles per XCD at a time)

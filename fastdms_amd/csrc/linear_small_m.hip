@@ -913,7 +913,7 @@ __global__ __launch_bounds__(NW * 64) void linear_small_m_kernel(
     }
     return;
   }
-  uint32_t vmax = 0;  // the row's max |output| over this strip, as abs_bits (rows >= M hold x = 0)
+  uint32_t vmax = 0;  // the row's max |output| over this strip, as abs_bits (rows >= M are not stored)
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int n = n0 + 4 * (lane >> 4) + r;

@@ -120,21 +120,22 @@ __device__ __forceinline__ bf16x8 read_v(uint32_t at, int row_bytes) {
 // K/V blocks go from global memory straight into LDS (the lane picks which
 // chunk it loads, see the swizzles above), double-buffered.
 //
-// What bounds it: power and the matrix cores together -- the clock falls to
-// 1.8 GHz while it runs (2.35 GHz under a memory-bound kernel) with the matrix
-// cores 51 % (head_dim 64) / 59 % (128) and the VALU 73 % / 46 % busy -- so what
+// What bounds it: the matrix cores are 51 % (head_dim 64) / 59 % (128) and the
+// VALU 72 % / 47 % busy, without LDS bank conflicts, at a clock that falls to
+// 1.5-1.8 GHz (2.3-2.5 GHz under the memory-bound kernels of the same run; all
+// from counters), and variants that only move work around change little, so what
 // counts is work per score.  32 rows per wave in 32x32 tiles keep two waves per
 // SIMD at head_dim 128 and three at 64 (227 / 159 VGPRs); the direct LDS loads
 // and the transposing reads take the V transposition and the staging registers
 // away, one lane per query the softmax broadcasts, and v_dot2 the extra P . 1
-// tile.  Measured against 16x16 tiles staged through registers: eight ragged
-// prompts of 6 144 tokens, 32 / 8 heads, head_dim 64 1 670 -> 1 380 us (929
-// TFLOP/s), head_dim 128 3 197 -> 2 428 us (1 059); 4 096 queries over a 12 300
-// token prefix, head_dim 128 1 128 -> 854 us (1 134); 24 prompts of 400 tokens
-// 46 -> 34.6 us.  P.V delayed by a block (so that one straight-line region holds
-// both products and the exponentials) measured +2 % / -0.5 %, and replacing
-// the per-block max by a check of the running sum -2.7 % at head_dim 64 but +1 to
-// +5 % at 128.
+// tile.  Measured against 16x16 tiles staged through registers (both in turn on
+// one card; cards differ by a tenth): eight ragged prompts of 6 144 tokens on
+// average, 32 / 8 heads, head_dim 64 1 690 -> 1 390 us (968 TFLOP/s), head_dim 128
+// 3 197 -> 2 435 us (1 104); 4 096 queries over a 12 300 token prefix, head_dim 128
+// 1 099 -> 843 us (1 142); 24 prompts of 400 tokens 46 -> 37 us.
+// P.V delayed by a block (so that one straight-line region holds both products
+// and the exponentials) measured +2 % / -0.5 %, and replacing the per-block max by
+// a check of the running sum -2.7 % at head_dim 64 but +1 to +5 % at 128.
 //
 // Software pipeline over the blocks: iteration t holds S of block t, issues
 // the loads of K(t + 2) and V(t + 1), multiplies K(t + 1) . Q^T beside the
@@ -435,8 +436,8 @@ FDMS_EXPORT int fdms_prefill_attention_varlen(const void* q, int64_t qs_t, int64
   const int vec_out = ((uintptr_t)out % 16) == 0 && os_t % 8 == 0 && os_h % 8 == 0;
   const dim3 grid((unsigned)((max_seqlen_q + pos - 1) / pos), (unsigned)(num_q_heads / packed), (unsigned)num_seqs);
 #define FDMS_PREFILL(DD, ...)                                                                                      \
-  hipLaunchKernelGGL((prefill_attn_kernel<DD, __VA_ARGS__>), grid, dim3(kThreads), 0, (hipStream_t)stream, (const bf16_t*)q,  \
-                     qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h, (bf16_t*)out, os_t,     \
+  hipLaunchKernelGGL((prefill_attn_kernel<DD, __VA_ARGS__>), grid, dim3(kThreads), 0, (hipStream_t)stream,            \
+                     (const bf16_t*)q, qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h, (bf16_t*)out, os_t,     \
                      os_h, cu_seqlens_q, cu_seqlens_k, group, vec_out, sl2, q_sign, max_floor)
 #define FDMS_PREFILL_GROUP(DD)                                                                                     \
   do {                                                                                                             \

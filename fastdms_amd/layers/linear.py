@@ -510,11 +510,15 @@ def linear_int4_partials(x: torch.Tensor, packed: torch.Tensor, scale_zeros: tor
 def fp8_gemm_impl() -> str:
     """The FP8 GEMM of prefill row counts: "hipblaslt" (default; torch's
     _scaled_mm with row-wise scales, the call the reference makes in
-    _fp8_linear, linear.py:652-659: a plain library GEMM, 1.8-2.2 PFLOP/s at
-    the Llama-3.2-1B prefill shapes on MI355X) or "fdms" (fdms_fp8_gemm, this
-    library's FP8 matrix-core kernel, 1.2-2.0 PFLOP/s there).
-    FASTDMS_AMD_FP8_GEMM selects; shapes hipBLASLt does not take (K or N not
-    multiples of 16) run fdms_fp8_gemm, row counts are padded to 16."""
+    _fp8_linear, linear.py:652-659: a plain library GEMM) or "fdms"
+    (fdms_fp8_gemm, this library's FP8 matrix-core kernel).  On MI355X, with the
+    row quantisation in front: at 43 864 rows of the Llama-3.2-1B shapes the
+    library reaches 1.6-2.2 PFLOP/s and fdms_fp8_gemm 1.4-1.8 (qkv 350 / 373 us,
+    gate_up 1 354 / 1 620, down 851 / 888), at 8 192 rows of the Qwen3-8B shapes
+    2.2-2.5 and 1.9-2.0; below about 2 000 rows fdms_fp8_gemm is the faster (300 x
+    16384 x 2048 56 / 27 us, 1500 x 4096 x 4096 57 / 45).  FASTDMS_AMD_FP8_GEMM
+    selects; shapes hipBLASLt does not take (K or N not multiples of 16) run
+    fdms_fp8_gemm, row counts are padded to 16."""
     impl = os.environ.get("FASTDMS_AMD_FP8_GEMM", "hipblaslt").strip().lower()
     if impl not in ("hipblaslt", "fdms"):
         raise ValueError(f"FASTDMS_AMD_FP8_GEMM must be 'hipblaslt' or 'fdms', got {impl!r}")
@@ -527,9 +531,10 @@ def fp8_gemm(x: torch.Tensor, weight_fp8: torch.Tensor, weight_scale_inv: torch.
     """_fp8_linear for prefill row counts on the FP8 matrix cores
     (linear.py:635-662): rows quantised per row (fdms_quantize_fp8_rows), then
     y = bf16(sum_k xq * w8 * x_scale_inv * w_scale_inv) with fp32 accumulation
-    (fp8_gemm_impl: hipBLASLt's scaled GEMM or fdms_fp8_gemm), bias added in
-    bf16.  x [M, K] bf16 / fp32, weight_fp8 [N, K] e4m3fn, K a multiple of
-    16."""
+    (``impl``, by default fp8_gemm_impl(): hipBLASLt's scaled GEMM or
+    fdms_fp8_gemm), bias added in bf16.  With ``out`` (bf16 [M, N], contiguous
+    columns) fdms_fp8_gemm writes into it whatever ``impl`` says.  x [M, K] bf16 /
+    fp32, weight_fp8 [N, K] e4m3fn, K a multiple of 16."""
     if x.dim() != 2 or weight_fp8.dim() != 2 or x.shape[1] != weight_fp8.shape[1]:
         raise ValueError(f"fp8_gemm shape mismatch: x {tuple(x.shape)}, weight {tuple(weight_fp8.shape)}")
     rows, k = x.shape

@@ -264,8 +264,9 @@ int fdms_record_dms_decisions(int32_t* positions, int64_t p_l, int64_t p_s, int6
 
 /* B1 — dense causal prefill attention over a ragged batch (bf16, head_dim 64
  * or 128, GQA).  Replaces the reference's flash_attn_varlen_func(causal=True)
- * call (fastdms/layers/attention.py:85-92).  Rows are 16-byte aligned;
- * cu_seqlens [num_seqs+1] on the device; max_seqlen bounds the grid. */
+ * call (fastdms/layers/attention.py:85-92).  Rows are 16-byte aligned; scale
+ * of either sign or 0; cu_seqlens [num_seqs+1] on the device; max_seqlen bounds
+ * the grid. */
 int fdms_prefill_attention(const void* q, int64_t qs_t, int64_t qs_h, const void* k, int64_t ks_t, int64_t ks_h,
                            const void* v, int64_t vs_t, int64_t vs_h, void* out, int64_t os_t, int64_t os_h,
                            const int32_t* cu_seqlens, int num_seqs, int max_seqlen, int num_q_heads,
