@@ -136,18 +136,24 @@ def prefill_qk_supported(q: torch.Tensor, k: torch.Tensor, cos_sin_cache: torch.
     """Views that fdms_prefill_qk takes: bf16 rows of 64 or 128 values moved as
     16-byte vectors, at most 2 048 such vectors per token, fp32 cos / sin rows
     and norm weights as wide as a head (the kernel reads head_dim of each)."""
-    d = q.shape[2]
-    tensors = (q, k, cos_sin_cache) + tuple(n.weight for n in norms)
-    return (q.dtype == k.dtype == torch.bfloat16 and d in (64, 128) and q.shape[0] > 0
-            and k.shape[0] == q.shape[0] and k.shape[2] == d
-            and q.shape[1] % k.shape[1] == 0 and (q.shape[1] + k.shape[1]) * d // 8 <= 2048
-            and q.stride(2) == k.stride(2) == 1
-            and all(s % 8 == 0 for s in (q.stride(0), q.stride(1), k.stride(0), k.stride(1)))
-            and cos_sin_cache.dtype == torch.float32 and cos_sin_cache.shape[2] == d and cos_sin_cache.stride(2) == 1
-            and cos_sin_cache.stride(0) % 4 == 0
-            and all(n.weight.dtype == torch.bfloat16 and n.weight.shape == (d,) and n.weight.is_contiguous()
-                    for n in norms)
-            and all(t.data_ptr() % 16 == 0 for t in tensors))
+    tokens, hq, d = q.shape
+    if d not in (64, 128) or tokens == 0 or q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16:
+        return False
+    k_tokens, hkv, k_d = k.shape
+    if k_tokens != tokens or k_d != d or hq % hkv or (hq + hkv) * d > 2048 * 8:
+        return False
+    (q_t, q_h, q_d), (k_t, k_h, k_d) = q.stride(), k.stride()
+    if q_d != 1 or k_d != 1 or (q_t | q_h | k_t | k_h) % 8 or (q.data_ptr() | k.data_ptr()) % 16:
+        return False
+    cs_p, _, cs_d = cos_sin_cache.stride()
+    if (cos_sin_cache.dtype != torch.float32 or cos_sin_cache.shape[2] != d or cs_d != 1 or cs_p % 4
+            or cos_sin_cache.data_ptr() % 16):
+        return False
+    for n in norms:
+        w = n.weight
+        if w.dtype != torch.bfloat16 or w.shape != (d,) or w.stride(0) != 1 or w.data_ptr() % 16:
+            return False
+    return True
 
 
 def prefill_qk_inplace(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor, cos_sin_cache: torch.Tensor, *,

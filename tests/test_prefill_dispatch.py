@@ -49,6 +49,42 @@ def test_prefill_qk_refuses_rows_it_would_read_past(what):
     assert not prefill_qk_supported(q, k, table, norms)
 
 
+
+@pytest.mark.parametrize("what", ["no tokens", "head width", "fp32 q", "fp16 k", "odd token stride", "odd head stride",
+                                  "odd offset", "strided dim", "heads", "lanes", "table type", "strided table",
+                                  "odd table rows", "norm type", "strided norm", "odd norm offset"])
+def test_prefill_qk_refuses_rows_it_cannot_move(what):
+    """Types, strides and alignments its 16-byte moves do not take."""
+    hq, hkv = (256, 16) if what == "lanes" else (4, 3) if what == "heads" else (HQ, HKV)
+    d = 32 if what == "head width" else D
+    tokens = 0 if what == "no tokens" else TOKENS
+    width = (hq + 2 * hkv) * d + (4 if what == "odd token stride" else 0)
+    store = torch.zeros(TOKENS * 2 * width + 16, dtype=torch.bfloat16)
+    offset = 4 if what == "odd offset" else 0
+    rows = store[offset:offset + tokens * width].view(tokens, width)
+    q, k = rows[:, :hq * d].view(-1, hq, d), rows[:, hq * d:(hq + hkv) * d].view(-1, hkv, d)
+    if what == "odd head stride":
+        q = store.as_strided((tokens, hq, d), (width, d + 4, 1))
+    if what == "strided dim":
+        k = store.as_strided((tokens, hkv, d), (2 * width, 2 * d, 2))
+    q = q.float() if what == "fp32 q" else q
+    k = k.half() if what == "fp16 k" else k
+    table = torch.zeros(16, 1, d)
+    if what == "table type":
+        table = table.double()
+    if what == "strided table":
+        table = torch.zeros(16, 1, 2 * d)[..., ::2]
+    if what == "odd table rows":
+        table = torch.zeros(16, 1, d + 2)[..., :d]
+    norms = _norms(d)
+    if what == "norm type":
+        norms[0].weight.data = norms[0].weight.data.float()
+    if what == "strided norm":
+        norms[1].weight.data = torch.ones(2 * d, dtype=torch.bfloat16)[::2]
+    if what == "odd norm offset":
+        norms[1].weight.data = torch.ones(d + 4, dtype=torch.bfloat16)[4:]
+    assert not prefill_qk_supported(q, k, table, norms)
+
 def _prefill(hooked=(), replace=None):
     """Prefill logits of a two-layer QK-norm model with forward hooks on the
     named modules of layer 1; returns (logits, hook calls, kernel calls)."""
