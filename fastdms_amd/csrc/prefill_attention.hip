@@ -437,8 +437,8 @@ FDMS_EXPORT int fdms_prefill_attention_varlen(const void* q, int64_t qs_t, int64
   const dim3 grid((unsigned)((max_seqlen_q + pos - 1) / pos), (unsigned)(num_q_heads / packed), (unsigned)num_seqs);
 #define FDMS_PREFILL(DD, ...)                                                                                      \
   hipLaunchKernelGGL((prefill_attn_kernel<DD, __VA_ARGS__>), grid, dim3(kThreads), 0, (hipStream_t)stream,            \
-                     (const bf16_t*)q, qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t, vs_h, (bf16_t*)out, os_t,     \
-                     os_h, cu_seqlens_q, cu_seqlens_k, group, vec_out, sl2, q_sign, max_floor)
+                     (const bf16_t*)q, qs_t, qs_h, (const bf16_t*)k, ks_t, ks_h, (const bf16_t*)v, vs_t,      \
+                     vs_h, (bf16_t*)out, os_t, os_h, cu_seqlens_q, cu_seqlens_k, group, vec_out, sl2, q_sign, max_floor)
 #define FDMS_PREFILL_GROUP(DD)                                                                                     \
   do {                                                                                                             \
     if (group == 1) FDMS_PREFILL(DD, 1, false); else if (group == 2) FDMS_PREFILL(DD, 2, false);                   \
